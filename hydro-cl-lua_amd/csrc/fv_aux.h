@@ -58,17 +58,17 @@ template <typename R, template <typename> class EQ, int DIM>
 __global__ void __launch_bounds__(256) dt_kernel(const GridArgs<R> g) {
 	using E = EQ<R>;
 	constexpr int Q = E::Q;
-	double m = INFINITY;
+	FastestWave<DIM> fw;
 	for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < g.ncell; c += (long)gridDim.x * blockDim.x) {
 		double u[Q + E::NSTAT];
 #pragma unroll
 		for (int j = 0; j < Q; ++j) u[j] = (double)g.U[j * g.ps + c];
 #pragma unroll
 		for (int j = 0; j < E::NSTAT; ++j) u[Q + j] = (double)g.stat[j * g.ps + c];
-		double d = E::template dt_cell<DIM>(g.pd, g.dx, u);
-		m = fmin(m, d);
+		E::template fastest<DIM>(g.pd, u, fw.lam);
+		fw.seen = true;
 	}
-	m = wave_min(m);
+	const double m = wave_min(fw.dt(g.dx));
 	int w = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
 	if ((threadIdx.x & 63) == 0 && m < INFINITY) atomic_min_pos(&g.dev->dtmin[g.slot][w & (DT_LANES - 1)], m);
 }
@@ -82,7 +82,7 @@ __global__ void __launch_bounds__(256) constrain_kernel(const GridArgs<R> g) {
 		double u[Q];
 #pragma unroll
 		for (int j = 0; j < Q; ++j) u[j] = (double)g.U[j * g.ps + c];
-		E::constrain(g.pd.gamma, g.pd.rhoMin, g.pd.PMin, u);
+		E::constrain(g.pd, u);
 #pragma unroll
 		for (int j = 0; j < Q; ++j) g.U[j * g.ps + c] = R(u[j]);
 	}

@@ -81,6 +81,7 @@ struct GridDesc {
 	int derivOn;              // volume > 1e-7 (fvsolver.cl:97)
 	int fluxOn[3];            // cell_area > 1e-7 (fvsolver.lua:105)
 	R aovFast[3];             // FAST kernels: areaOverVol where flux and derivative are on, else 0
+	R aovHalf[3];             // half of it, for the Roe form that returns twice the flux
 	R dx[3];
 	R invdx[3];               // 1 / dx in the stored precision (glm-maxwell.cl:351)
 	R inv2dx[3];              // 1 / (2 dx) in the stored precision (makepartial.lua:105-108)
@@ -100,6 +101,7 @@ struct GridDesc {
 // in every stored precision.
 struct EqnParD {
 	double gamma, rhoMin, PMin;   // Euler (euler.lua:192-197)
+	double eIntSafe;              // Euler: 2 PMin / (gamma - 1), the internal energy from which on P is above PMin
 	double divPhi, divPsi;        // GLM-Maxwell (glm-maxwell.lua:110-111)
 	double gravity;               // shallow water (shallow-water.lua:167)
 };
@@ -269,6 +271,27 @@ __device__ __forceinline__ void atomic_min_pos(double *p, double v) {
 	// positive doubles (and +inf) order like their bit patterns
 	atomicMin(reinterpret_cast<unsigned long long *>(p), (unsigned long long)__double_as_longlong(v));
 }
+
+// The CFL step of the cells a lane has seen, from the fastest wave of each axis
+// (calcDT.cl:38-73 takes the minimum of dx / max(1e-9, |lambda|) per cell and
+// axis): division is monotonic, so dx / max is the same minimum bit for bit,
+// with one division per axis and wave in place of one per axis and cell.
+template <int DIM>
+struct FastestWave {
+	double lam[DIM];
+	bool seen;
+	__device__ __forceinline__ FastestWave() : seen(false) {
+#pragma unroll
+		for (int s = 0; s < DIM; ++s) lam[s] = 0.;
+	}
+	__device__ __forceinline__ double dt(const double *dx) const {
+		double d = INFINITY;
+#pragma unroll
+		for (int s = 0; s < DIM; ++s)
+			if (dx[s] > 0.) d = fmin(d, dx[s] / fmax(1e-9, lam[s]));
+		return seen ? d : INFINITY;
+	}
+};
 
 // Logical block id with blocks spread so that each XCD (blocks are dealt
 // round-robin over the 8 XCDs) gets a contiguous range of logical ids, so

@@ -246,7 +246,7 @@ struct Eqn {
 		l[6] = p.divPhi; l[7] = p.divPsi;
 	}
 
-	__device__ static __forceinline__ void constrain(double, double, double, double *) {}
+	__device__ static __forceinline__ void constrain(const EqnParD &, double *) {}
 
 	// addSource (glm-maxwell.cl:317-380) for one interior cell: U the cell's
 	// cons_t, em / ep the sqrt_1_eps of its -1 / +1 neighbours per axis. The
@@ -300,22 +300,12 @@ struct Eqn {
 		d[6] = d[6] + U[8] * p.divPhi;
 	}
 
-	// calcDTCell with the GLM wave bounds (glm-maxwell.lua:216-245)
+	// the GLM wave bounds per axis (glm-maxwell.lua:216-245)
 	template <int DIM>
-	__device__ static __forceinline__ double dt_cell(const EqnParD &pd, const double *dx, const double *U) {
-		using MD = Math<double, FAST>;
-		const double divPhi = pd.divPhi, divPsi = pd.divPsi;
-		double dt = INFINITY;
-		for (int s = 0; s < DIM; ++s) {
-			if (dx[s] > 0.) {
-				double v_p_abs = U[10] * U[11] * (1. / 1.);
-				double wmax = fmax(fmax(divPsi, divPhi), v_p_abs);
-				double absLambdaMax = fmax(fabs(wmax), fabs(-wmax));
-				absLambdaMax = fmax(1e-9, absLambdaMax);
-				dt = fmin(dt, MD::div(dx[s], absLambdaMax));
-			}
-		}
-		return dt;
+	__device__ static __forceinline__ void fastest(const EqnParD &pd, const double *U, double *lam) {
+		const double wmax = fmax(fmax(pd.divPsi, pd.divPhi), U[10] * U[11] * (1. / 1.));
+#pragma unroll
+		for (int s = 0; s < DIM; ++s) lam[s] = fmax(lam[s], fabs(wmax));
 	}
 
 	// mirror reflects D and B along the axis (reflectVars.mirror, eqn.lua:366-370)

@@ -61,6 +61,7 @@ static inline EqnParD eqn_par_d(const hydro_cfg &c) {
 	p.gamma = c.gamma;
 	p.rhoMin = c.rho_min;
 	p.PMin = c.P_min;
+	p.eIntSafe = 2. * c.P_min / (c.gamma - 1.);
 	p.divPhi = c.div_phi_wavespeed;
 	p.divPsi = c.div_psi_wavespeed;
 	p.gravity = c.gravity;
@@ -445,6 +446,7 @@ static void grid_desc(const Grid &g, GridDesc<R> &d) {
 		// both guards as one factor: the flux term is then exactly 0 where a
 		// guard is off (for finite fluxes; the sign of a zero may differ)
 		d.aovFast[side] = d.fluxOn[side] && d.derivOn ? d.areaOverVol[side] : R(0);
+		d.aovHalf[side] = R(.5) * d.aovFast[side];
 	}
 	d.cfl = c.cfl;
 	d.rowsPerWave = g.rowsPerWave;

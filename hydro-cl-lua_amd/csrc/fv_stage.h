@@ -499,7 +499,8 @@ __host__ __device__ constexpr bool redo_form(bool lim) {
 // speed is the right state's: the reference assigns it per side in turn), or
 // HLLC (euler-hllc.cl:13-240, hllcMethod 2, HLL's estimates), or Marquina
 // (marquina.cl:5-93). The cases of HLL and HLLC are selects over all
-// candidate fluxes, in the reference's expression order each.
+// candidate fluxes, in the reference's expression order each. Where the Roe
+// flux has a collected form, F is twice the flux (flux_aov carries the half).
 template <typename R, class E, int S, int RM = ROE_INLINE>
 __device__ __forceinline__ void iface_solve(const typename E::Par &p, const Cell<R, E> &UL, const Cell<R, E> &UR,
 	R dt_dx, int lim, R *F, bool *ok = nullptr)
@@ -516,6 +517,10 @@ __device__ __forceinline__ void iface_solve(const typename E::Par &p, const Cell
 		Iface<R, E> I;
 		iface_prep_general<R, E, S>(p, UL, UR, I);
 		iface_flux<R, E, S, false, 0>(p, I, nullptr, nullptr, dt_dx, lim, F);
+		if constexpr (roe_collected<E>(false)) {
+#pragma unroll
+			for (int j = 0; j < E::Q; ++j) F[j] = R(2) * F[j];     // as the collected form's
+		}
 	} else {
 		using M = typename E::M;
 		auto WL = E::prim(p, UL.v);
@@ -622,14 +627,15 @@ __device__ __forceinline__ void iface_solve(const typename E::Par &p, const Cell
 // The reference zeroes a flux where the cell area is <= 1e-7 and the whole
 // derivative where the volume is (fvsolver.lua:105, fvsolver.cl:97). EXACT
 // kernels apply both as selects; FAST kernels fold them into one factor per
-// side (GridDesc::aovFast), one multiply and no selects.
+// side (GridDesc::aovFast), one multiply and no selects. The collected Roe
+// form returns twice the flux: its factor is half as large (exact).
 template <class E, typename R>
 __device__ __forceinline__ bool flux_on(const GridDesc<R> &g, int side) {
 	return E::FASTM ? true : g.fluxOn[side] != 0;
 }
-template <class E, typename R>
+template <class E, bool LIM, typename R>
 __device__ __forceinline__ R flux_aov(const GridDesc<R> &g, int side) {
-	return E::FASTM ? g.aovFast[side] : g.areaOverVol[side];
+	return roe_collected<E>(LIM) ? g.aovHalf[side] : E::FASTM ? g.aovFast[side] : g.areaOverVol[side];
 }
 
 // ------------------------------------------------------------ strip edges
@@ -825,7 +831,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 	const typename E::Par par = E::par(a);
 	const int lim = PLM ? 0 : a.limiter;   // runtime limiter index when FLIM/SLIM == -1
 	const int slim = a.limiter;
-	double dtLocal = INFINITY;
+	FastestWave<DIM> fw;     // of the new state, on the last stage
 
 	const int nx = g.n[0];
 	const int ny = DIM >= 2 ? g.n[1] : 1;
@@ -881,7 +887,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 				R Fa[Q], dW[E::NW];
 				bool ok;
 				edge_flux<R, E, PLM, LIM, FLIM, SLIM, RM>(par, lim, slim, cb, dt_dx0, flux_on<E>(g, 0),
-					flux_aov<E>(g, 0), Fa, dW, ok);
+					flux_aov<E, LIM>(g, 0), Fa, dW, ok);
 				edges[0].ok[lane] = ok ? 1 : 0;
 #pragma unroll
 				for (int q = 0; q < Q; ++q) edges[0].fa[q][lane] = Fa[q];
@@ -920,7 +926,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 				for (int k = 0; k < 4; ++k) load_cell<R, E>(g, src, mxb[k], myb, cb[k]);
 			}
 			edge_pass<R, E, PLM, LIM, FLIM, SLIM, EDGE_ROWS, RM>(par, lim, slim, cb, dt_dx0, flux_on<E>(g, 0),
-				flux_aov<E>(g, 0), lane, edge);
+				flux_aov<E, LIM>(g, 0), lane, edge);
 		}
 	}
 
@@ -997,7 +1003,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 			}
 #pragma unroll
 			for (int j = 0; j < Q; ++j) {
-				R FaY = flux_on<E>(g, 1) ? F[j] * flux_aov<E>(g, 1) : R(0);
+				R FaY = flux_on<E>(g, 1) ? F[j] * flux_aov<E, LIM>(g, 1) : R(0);
 				dyterm[j] = FaY - FaYprev[j];
 				FaYprev[j] = FaY;
 			}
@@ -1013,7 +1019,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 			bool okX;
 			const int jr = r - y0;
 			strip_x<R, E, PLM, LIM, FLIM, SLIM, EDGE_ROWS, EDGES, RM>(par, lim, slim, U, dt_dx0, flux_on<E>(g, 0),
-				flux_aov<E>(g, 0), lane, share ? w * rpw + jr : jr, share ? (w + 1) * rpw + jr : EDGE_ROWS + jr, edge,
+				flux_aov<E, LIM>(g, 0), lane, share ? w * rpw + jr : jr, share ? (w + 1) * rpw + jr : EDGE_ROWS + jr, edge,
 				edgeR, Um, Up, deriv, okX);
 			if constexpr (RM == ROE_FLAGGED) {
 				// an irregular interface of this row: the redo kernel takes the
@@ -1076,7 +1082,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 					for (int j = 0; j < Q; ++j)
 						if (E::active(j)) acc[j] = acc[j] + (double)deriv[j] * c;
 				}
-				E::constrain(a.pd.gamma, a.pd.rhoMin, a.pd.PMin, acc);
+				E::constrain(a.pd, acc);
 				R o[Q];
 #pragma unroll
 				for (int j = 0; j < Q; ++j) {
@@ -1089,8 +1095,8 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 					for (int j = 0; j < Q; ++j) ud[j] = (double)o[j];
 #pragma unroll
 					for (int j = Q; j < C::NV; ++j) ud[j] = (double)U.v[j];
-					double d = E::template dt_cell<DIM>(a.pd, g.dxD, ud);
-					dtLocal = fmin(dtLocal, d);
+					E::template fastest<DIM>(a.pd, ud, fw.lam);
+					fw.seen = true;
 				}
 			}
 		}
@@ -1104,7 +1110,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 		}
 	}
 	}
-	return dtLocal;
+	return a.reduceSlot >= 0 ? fw.dt(g.dxD) : INFINITY;
 }
 
 // dt of this step for grid g (solverbase.lua:3016): cfl * min, or a host value
@@ -1139,8 +1145,17 @@ __device__ __forceinline__ void stage_reduce(const StageArgs<R> &a, const GridDe
 // equations with the Roe flux and no flux limiter take the collected Roe form
 // only (ROE_FLAGGED) and leave any strip with an irregular interface, from
 // that row on, to stage_kernel_redo, launched after them on the same stream.
+// The FP64 form of 'plm cons' or no reconstruction without an out-of-plane
+// velocity needs about 128 registers, the most that lets a SIMD hold four
+// waves: it is held to that (the allocator takes 130 on its own, three waves).
+template <typename R, class E, int DIM>
+__host__ __device__ constexpr int plain_min_blocks(bool lim) {
+	return sizeof(R) == 8 && redo_form<E, DIM>(lim) && !E::active(3) && !E::PLM_PRIM && !E::PLM_EIG && !E::PLM_CONS_FLUX
+		&& !E::PLM_ATHENA && !E::PLM_PPM && !E::PLM_EIG_PRIM && !E::PLM_EIG_PRIM_REF ? 4 : 1;
+}
+
 template <typename R, template <typename> class EQ, int DIM, bool PLM, bool LIM, int FLIM, int SLIM>
-__global__ void __launch_bounds__(256) stage_kernel(const StageArgs<R> a)
+__global__ void __launch_bounds__(256, (plain_min_blocks<R, EQ<R>, DIM>(LIM))) stage_kernel(const StageArgs<R> a)
 {
 	constexpr int RM = redo_form<EQ<R>, DIM>(LIM) ? ROE_FLAGGED : ROE_INLINE;
 	const int lane = threadIdx.x & 63;

@@ -99,7 +99,7 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 	const typename E::Par par = E::par(a);
 	const int lim = PLM ? 0 : a.limiter;
 	const int slim = a.limiter;
-	double dtLocal = INFINITY;
+	FastestWave<3> fw;     // of the new state, on the last stage
 
 	const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
 	const R *src = g.U[a.src];
@@ -152,7 +152,7 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 			for (int k = 0; k < 4; ++k) load_cell3<R, E>(g, src, mxb[k], myOwn, mz, cb[k]);
 		}
 		edge_pass<R, E, PLM, LIM, FLIM, SLIM, EDGE_PLANES>(par, lim, slim, cb, dt_dx0, flux_on<E>(g, 0),
-			flux_aov<E>(g, 0), lane, edge);
+			flux_aov<E, LIM>(g, 0), lane, edge);
 	}
 
 	// z pipeline state (the 2D kernel's y pipeline)
@@ -222,7 +222,7 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 			}
 #pragma unroll
 			for (int j = 0; j < Q; ++j) {
-				R FaZ = flux_on<E>(g, 2) ? F[j] * flux_aov<E>(g, 2) : R(0);
+				R FaZ = flux_on<E>(g, 2) ? F[j] * flux_aov<E, LIM>(g, 2) : R(0);
 				dzterm[j] = FaZ - FaZprev[j];
 				FaZprev[j] = FaZ;
 			}
@@ -264,7 +264,7 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 			R FaY[Q];
 #pragma unroll
 			for (int j = 0; j < Q; ++j) {
-				FaY[j] = flux_on<E>(g, 1) ? Fy[j] * flux_aov<E>(g, 1) : R(0);
+				FaY[j] = flux_on<E>(g, 1) ? Fy[j] * flux_aov<E, LIM>(g, 1) : R(0);
 				sh.f[w][j][lane] = FaY[j];
 			}
 			__syncthreads();
@@ -277,7 +277,7 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 			R deriv[Q];
 			bool okx;   // unused: the 3D kernel takes the general Roe form where an interface is irregular (ROE_INLINE)
 			strip_x<R, E, PLM, LIM, FLIM, SLIM, EDGE_PLANES>(par, lim, slim, U, dt_dx0, flux_on<E>(g, 0),
-				flux_aov<E>(g, 0), lane, r - z0, EDGE_PLANES + (r - z0), edge, edge, Um, Up, deriv, okx);
+				flux_aov<E, LIM>(g, 0), lane, r - z0, EDGE_PLANES + (r - z0), edge, edge, Um, Up, deriv, okx);
 #pragma unroll
 			for (int j = 0; j < Q; ++j) {
 				deriv[j] = deriv[j] - dyterm[j];
@@ -320,7 +320,7 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 					for (int j = 0; j < Q; ++j)
 						if (E::active(j)) acc[j] = acc[j] + (double)deriv[j] * c;
 				}
-				E::constrain(a.pd.gamma, a.pd.rhoMin, a.pd.PMin, acc);
+				E::constrain(a.pd, acc);
 				R o[Q];
 #pragma unroll
 				for (int j = 0; j < Q; ++j) {
@@ -333,8 +333,8 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 					for (int j = 0; j < Q; ++j) ud[j] = (double)o[j];
 #pragma unroll
 					for (int j = Q; j < NV; ++j) ud[j] = (double)U.v[j];
-					double d = E::template dt_cell<3>(a.pd, g.dxD, ud);
-					dtLocal = fmin(dtLocal, d);
+					E::template fastest<3>(a.pd, ud, fw.lam);
+					fw.seen = true;
 				}
 			}
 		}
@@ -344,7 +344,7 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 		else { W0 = W1; }
 	}
 	}
-	return dtLocal;
+	return a.reduceSlot >= 0 ? fw.dt(g.dxD) : INFINITY;
 }
 
 // The halo wave of the block: per output plane, the rows y0-2, y0-1 and
@@ -438,7 +438,7 @@ __device__ __forceinline__ void stage_halo3d(const StageArgs<R> &a, const GridDe
 			__syncthreads();
 		}
 #pragma unroll
-		for (int j = 0; j < Q; ++j) sh.f[W][j][lane] = flux_on<E>(g, 1) ? F[j] * flux_aov<E>(g, 1) : R(0);
+		for (int j = 0; j < Q; ++j) sh.f[W][j][lane] = flux_on<E>(g, 1) ? F[j] * flux_aov<E, LIM>(g, 1) : R(0);
 		__syncthreads();
 	}
 }

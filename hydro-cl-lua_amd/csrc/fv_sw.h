@@ -221,7 +221,7 @@ struct Eqn {
 		l[3] = v_n + C_nLen;
 	}
 
-	__device__ static __forceinline__ void constrain(double, double, double, double *) {}
+	__device__ static __forceinline__ void constrain(const EqnParD &, double *) {}
 
 	// addSource (shallow-water.cl:366-428, its enabled block) for one interior
 	// cell: em / ep the depth of the -1 / +1 neighbours per axis; the
@@ -244,31 +244,24 @@ struct Eqn {
 		}
 	}
 
-	// calcDTCell (calcDT.cl:38-73) with consWaveCodeMinMaxAllSides
-	// (shallow-water.lua:318-354), in double
+	// the state's fastest wave per axis (calcDT.cl:38-73 with
+	// consWaveCodeMinMaxAllSides, shallow-water.lua:318-354), in double
 	template <int DIM>
-	__device__ static __forceinline__ double dt_cell(const EqnParD &pd, const double *dx, const double *U) {
+	__device__ static __forceinline__ void fastest(const EqnParD &pd, const double *U, double *lam) {
 		using MD = Math<double, FAST>;
 		const double CSq = pd.gravity * U[0];
 		const double C = MD::sqrt_(CSq);
 		const double inv = MD::rcp(U[0]);
-		double dt = INFINITY;
 #pragma unroll
 		for (int s = 0; s < DIM; ++s) {
-			if (dx[s] > 0.) {
-				double C_nLen = C * 1.;
-				double v_n = U[1 + s] * inv;
-				if (C <= 0.) {
-					C_nLen = 0.;
-					v_n = 0.;
-				}
-				const double lmin = v_n - C_nLen, lmax = v_n + C_nLen;
-				double absLambdaMax = fmax(fabs(lmin), fabs(lmax));
-				absLambdaMax = fmax(1e-9, absLambdaMax);
-				dt = fmin(dt, MD::div(dx[s], absLambdaMax));
+			double C_nLen = C * 1.;
+			double v_n = U[1 + s] * inv;
+			if (C <= 0.) {
+				C_nLen = 0.;
+				v_n = 0.;
 			}
+			lam[s] = fmax(lam[s], fabs(v_n) + C_nLen);
 		}
-		return dt;
 	}
 
 	// mirror reflects the momentum along the axis (reflectVars.mirror, eqn.lua:366-370)
