@@ -17,7 +17,7 @@ struct GridArgs {
 	long ps;         // plane stride
 	long ncell;      // interior cells (planes are dense)
 	int dim;
-	double dx[3];
+	CflScale cflScale;
 	EqnParD pd;
 	DevScalars *dev;
 	int slot;
@@ -58,17 +58,18 @@ template <typename R, template <typename> class EQ, int DIM>
 __global__ void __launch_bounds__(256) dt_kernel(const GridArgs<R> g) {
 	using E = EQ<R>;
 	constexpr int Q = E::Q;
-	FastestWave<DIM> fw;
+	FastestWave<DIM, E::FASTM> fw;
 	for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < g.ncell; c += (long)gridDim.x * blockDim.x) {
 		double u[Q + E::NSTAT];
 #pragma unroll
 		for (int j = 0; j < Q; ++j) u[j] = (double)g.U[j * g.ps + c];
 #pragma unroll
 		for (int j = 0; j < E::NSTAT; ++j) u[Q + j] = (double)g.stat[j * g.ps + c];
-		E::template fastest<DIM>(g.pd, u, fw.lam);
-		fw.seen = true;
+		double lam[DIM];
+		E::template fastest<DIM>(g.pd, u, lam);
+		fw.add(g.cflScale, lam);
 	}
-	const double m = wave_min(fw.dt(g.dx));
+	const double m = wave_min(fw.dt(g.cflScale));
 	int w = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
 	if ((threadIdx.x & 63) == 0 && m < INFINITY) atomic_min_pos(&g.dev->dtmin[g.slot][w & (DT_LANES - 1)], m);
 }

@@ -50,10 +50,8 @@ struct DevScalars {
 	double dtmin[3][DT_LANES];
 	double t;
 	double dt;
-	unsigned redoCount;       // entries of the redo list of the running stage
-	unsigned redoDone;        // blocks of the redo kernel that have finished
 	unsigned nonFinite;       // set by nonfinite_kernel
-	unsigned pad0;
+	unsigned pad0[3];
 	double pad[4];
 };
 
@@ -61,6 +59,13 @@ struct DevScalars {
 struct AxisBC {
 	int n;            // interior cells
 	int kind[2];      // HYDRO_BC_* at min / max
+};
+
+// Cell lengths as the CFL step takes them (FastestWave)
+struct CflScale {
+	double dx[3];      // cell lengths
+	double len;        // the first positive one, INFINITY if there is none
+	double scale[3];   // len / dx, 0 for an axis that counts for nothing
 };
 
 // Everything that is specific to one grid: its buffers, shape, boundaries,
@@ -85,14 +90,13 @@ struct GridDesc {
 	R dx[3];
 	R invdx[3];               // 1 / dx in the stored precision (glm-maxwell.cl:351)
 	R inv2dx[3];              // 1 / (2 dx) in the stored precision (makepartial.lua:105-108)
-	double dxD[3];
+	CflScale cflScale;
 	double cfl;
 	int stripsX, stripsY, rowsPerWave;   // 3D: stripsY counts blocks of Block3::W rows, rowsPerWave planes per chunk
 	int active;               // batch: grid takes part in the launch
 	long itemBase;            // batch: first work item (wave strip) of this grid
 	long nItems;              // stripsX * stripsY
 	DevScalars *dev;          // dt slots and time of this grid
-	int2 *redo;               // redo list: (strip item, first row) per strip, at most one each
 	int stepsLeft;            // batch: steps still to run in the current tick
 	int stripsZ;              // 3D: plane chunks of rowsPerWave planes
 };
@@ -126,7 +130,6 @@ struct StageArgs {
 	int resetSlot;            // slot to clear to +inf, -1 none
 	int reduceSlot;           // slot to min-reduce the new state's dt into, -1 none
 	int advanceTime;          // t += dt, dt stored
-	int redoPass;             // this launch is the redo kernel of the stage
 	int shareEdges;           // plain 2D launch: one strip-edge pass per block of 4 x-adjacent strips
 	int stepInTick;           // batch: skip grids with stepsLeft <= stepInTick
 	// equation parameters in the stencil type and in double (for the FP64
@@ -272,23 +275,40 @@ __device__ __forceinline__ void atomic_min_pos(double *p, double v) {
 	atomicMin(reinterpret_cast<unsigned long long *>(p), (unsigned long long)__double_as_longlong(v));
 }
 
-// The CFL step of the cells a lane has seen, from the fastest wave of each axis
-// (calcDT.cl:38-73 takes the minimum of dx / max(1e-9, |lambda|) per cell and
-// axis): division is monotonic, so dx / max is the same minimum bit for bit,
-// with one division per axis and wave in place of one per axis and cell.
-template <int DIM>
+// The CFL step of the cells a lane has seen (calcDT.cl:38-73: the minimum of
+// dx / max(1e-9, |lambda|) over cells and axes) from the fastest wave: division
+// is monotonic, so dx / max is the minimum, with one division per wave in place
+// of one per axis and cell. The EXACT kernels keep the fastest wave of each
+// axis, whose dx / max is the reference's minimum bit for bit; the FAST ones
+// keep one value, every axis' waves scaled to the first axis' cell length (an
+// exact 1 where the lengths are equal): two registers less through the row loop.
+template <int DIM, bool FAST>
 struct FastestWave {
-	double lam[DIM];
+	static constexpr int N = FAST ? 1 : DIM;
+	double lam[N];
 	bool seen;
 	__device__ __forceinline__ FastestWave() : seen(false) {
 #pragma unroll
-		for (int s = 0; s < DIM; ++s) lam[s] = 0.;
+		for (int s = 0; s < N; ++s) lam[s] = 0.;
 	}
-	__device__ __forceinline__ double dt(const double *dx) const {
-		double d = INFINITY;
+	// l: a cell's fastest wave per axis
+	__device__ __forceinline__ void add(const CflScale &c, const double *l) {
 #pragma unroll
-		for (int s = 0; s < DIM; ++s)
-			if (dx[s] > 0.) d = fmin(d, dx[s] / fmax(1e-9, lam[s]));
+		for (int s = 0; s < DIM; ++s) {
+			if constexpr (FAST) lam[0] = fmax(lam[0], fmax(1e-9, l[s]) * c.scale[s]);
+			else lam[s] = fmax(lam[s], l[s]);
+		}
+		seen = true;
+	}
+	__device__ __forceinline__ double dt(const CflScale &c) const {
+		double d = INFINITY;
+		if constexpr (FAST) {
+			d = c.len / lam[0];
+		} else {
+#pragma unroll
+			for (int s = 0; s < DIM; ++s)
+				if (c.dx[s] > 0.) d = fmin(d, c.dx[s] / fmax(1e-9, lam[s]));
+		}
 		return seen ? d : INFINITY;
 	}
 };

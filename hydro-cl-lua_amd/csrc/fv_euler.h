@@ -559,7 +559,7 @@ struct EulerT {
 #pragma unroll
 			for (int s = 0; s < DIM; ++s) {
 				double vn = U[0] < rhoMin ? 0. : (s < NVEL ? MD::div_inv(U[1 + s], U[0], inv) : 0.);
-				lam[s] = fmax(lam[s], fabs(vn) + Cs);
+				lam[s] = fabs(vn) + Cs;
 			}
 		}
 

@@ -305,7 +305,7 @@ struct Eqn {
 	__device__ static __forceinline__ void fastest(const EqnParD &pd, const double *U, double *lam) {
 		const double wmax = fmax(fmax(pd.divPsi, pd.divPhi), U[10] * U[11] * (1. / 1.));
 #pragma unroll
-		for (int s = 0; s < DIM; ++s) lam[s] = fmax(lam[s], fabs(wmax));
+		for (int s = 0; s < DIM; ++s) lam[s] = fabs(wmax);
 	}
 
 	// mirror reflects D and B along the axis (reflectVars.mirror, eqn.lua:366-370)

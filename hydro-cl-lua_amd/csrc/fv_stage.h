@@ -469,14 +469,16 @@ __device__ __forceinline__ void iface_flux(const typename E::Par &p, const Iface
 // form where the interface is regular and the general form (every branch of
 // eigen_forInterface and the transforms) where it is not; ROE_FLAGGED takes
 // the collected form only and reports per lane whether the interface is
-// regular, so that the stage kernel leaves a strip from its first row with an
-// irregular interface on to the redo kernel (stage_kernel_redo), which runs
-// ROE_INLINE (1D and 3D kernels take ROE_INLINE throughout). Either way each
-// interface's form depends on its own states only, so a grid advances to the
-// same bits whatever its strips' heights and whether it runs alone or
-// batched. Keeping the general form out of the 2D stage kernel keeps its
-// registers at the collected form's (127 VGPRs FP64: 4 waves per SIMD,
-// against 186 with both forms).
+// regular, so that the wave leaves its row loop at the first row with an
+// irregular interface and does the rest of its strip cell by cell, each cell's
+// four interfaces from cells of its own loading (face_difference, ROE_INLINE).
+// Either way each interface's form depends on its own states only, so a grid
+// advances to the same bits whatever its strips' heights and whether it runs
+// alone or batched. With both forms in the row loop the FP64 kernel needs 186
+// VGPRs (2 waves per SIMD) in place of 128 (4); after the loop, with nothing
+// of its pipeline alive, the general form fits in what the loop has. (A second
+// launch per stage used to finish such strips: 2.7 us even when there was
+// none.)
 enum { ROE_GENERAL = 0, ROE_INLINE = 1, ROE_FLAGGED = 2 };
 
 template <class E>
@@ -484,11 +486,11 @@ __host__ __device__ constexpr bool roe_collected(bool lim) {
 	return E::FASTM && E::FLUXID == HYDRO_FLUX_ROE && E::Q == 5 && E::NW == 5 && !lim;
 }
 
-// The stage kernels that take ROE_FLAGGED and a redo launch: 2D. A 1D strip
-// is one row, so the general form costs it few registers (94 VGPRs FP64
-// against 74) and saves a launch per stage; 1D kernels take ROE_INLINE.
+// The stage kernels that take ROE_FLAGGED: 2D. A 1D strip is one row, so the
+// general form costs it few registers (94 VGPRs FP64 against 74); 1D kernels
+// take ROE_INLINE.
 template <class E, int DIM>
-__host__ __device__ constexpr bool redo_form(bool lim) {
+__host__ __device__ constexpr bool flagged_form(bool lim) {
 	return roe_collected<E>(lim) && DIM == 2;
 }
 
@@ -816,14 +818,163 @@ __device__ __forceinline__ void strip_x(const typename E::Par &par, int lim, int
 	}
 }
 
+// ------------------------------------------------------------ one cell's end
+// Integrator combine of one cell in double (rk.lua:155-174, fe.lua:50),
+// constrainU, the store, and the new state's fastest waves on the last stage.
+template <typename R, class E, int DIM>
+__device__ __forceinline__ void finish_cell(const StageArgs<R> &a, const GridDesc<R> &g, long off, const Cell<R, E> &U,
+	const R *deriv, double dt, R *out, R *storeD, FastestWave<DIM, E::FASTM> &fw)
+{
+	constexpr int Q = E::Q;
+	double acc[Q];
+#pragma unroll
+	for (int j = 0; j < Q; ++j) acc[j] = 0.;
+	for (int k = 0; k < a.nAlpha; ++k) {
+		const bool fromSrc = a.accU[k] == a.src;
+		const R *Uk = g.U[a.accU[k]];
+		double al = a.alpha[k];
+#pragma unroll
+		for (int j = 0; j < Q; ++j) {
+			if (!E::active(j)) continue;
+			R u = fromSrc ? U.v[j] : Uk[j * g.ps + off];
+			acc[j] = acc[j] + (double)u * al;
+		}
+	}
+	for (int k = 0; k < a.nStoredD; ++k) {
+		const R *Dk = g.D[a.accD[k]];
+		double c = (double)R(a.beta[k] * dt);
+#pragma unroll
+		for (int j = 0; j < Q; ++j)
+			if (E::active(j)) acc[j] = acc[j] + (double)Dk[j * g.ps + off] * c;
+	}
+	if (storeD) {
+#pragma unroll
+		for (int j = 0; j < Q; ++j)
+			if (E::active(j)) storeD[j * g.ps + off] = deriv[j];
+	}
+	if (a.betaNew != 0.) {
+		double c = (double)R(a.betaNew * dt);
+#pragma unroll
+		for (int j = 0; j < Q; ++j)
+			if (E::active(j)) acc[j] = acc[j] + (double)deriv[j] * c;
+	}
+	E::constrain(a.pd, acc);
+	R o[Q];
+#pragma unroll
+	for (int j = 0; j < Q; ++j) {
+		o[j] = R(acc[j]);
+		if (E::active(j)) out[j * g.ps + off] = o[j];
+	}
+	if (a.reduceSlot >= 0) {
+		double ud[Cell<R, E>::NV];
+#pragma unroll
+		for (int j = 0; j < Q; ++j) ud[j] = (double)o[j];
+#pragma unroll
+		for (int j = Q; j < Cell<R, E>::NV; ++j) ud[j] = (double)U.v[j];
+		double lam[DIM];
+		E::template fastest<DIM>(a.pd, ud, lam);
+		fw.add(g.cflScale, lam);
+	}
+}
+
+// ------------------------------------------------------- rows of general form
+// The flux, times its area factor, of the interface between cells c[1] and
+// c[2] of a line along axis S: iface_solve of the same states as in the row
+// loop and the strip edges, with the form chosen per interface.
+template <typename R, class E, int S, bool PLM, int SLIM>
+__device__ __forceinline__ void line_flux(const typename E::Par &par, int slim, const Cell<R, E> *c, R dt_dx,
+	bool fluxOn, R aov, R *Fa)
+{
+	R F[E::Q];
+	if constexpr (PLM) {
+		Cell<R, E> L1, R1, L2, R2;
+		plm_cons<R, E, SLIM, S>(par, slim, c[0], c[1], c[2], L1, R1, dt_dx);
+		plm_cons<R, E, SLIM, S>(par, slim, c[1], c[2], c[3], L2, R2, dt_dx);
+		iface_solve<R, E, S, ROE_INLINE>(par, R1, L2, dt_dx, 0, F);
+	} else {
+		iface_solve<R, E, S, ROE_INLINE>(par, c[1], c[2], dt_dx, 0, F);
+	}
+#pragma unroll
+	for (int j = 0; j < E::Q; ++j) Fa[j] = fluxOn ? F[j] * aov : R(0);
+}
+
+// The difference of the fluxes on the two faces of this lane's cell (x, y)
+// along axis S, from cells loaded for this lane alone.
+template <typename R, class E, int S, bool PLM, int SLIM>
+__device__ __forceinline__ void face_difference(const typename E::Par &par, int slim, const GridDesc<R> &g,
+	const R *src, int x, int y, R dt_dx, R *d)
+{
+#pragma unroll 1
+	for (int side = 0; side < 2; ++side) {
+		Cell<R, E> c[4];
+#pragma unroll
+		for (int k = 0; k < 4; ++k) {
+			const int i = side + k - 2;
+			const Mapped mx = map_coord(S == 0 ? x + i : x, g.n[0], g.bc[0], g.bc[1], 0);
+			const Mapped my = map_coord(S == 1 ? y + i : y, g.n[1], g.bc[2], g.bc[3], 2);
+			load_cell<R, E>(g, src, mx, my, c[k]);
+		}
+		R Fa[E::Q];
+		line_flux<R, E, S, PLM, SLIM>(par, slim, c, dt_dx, flux_on<E>(g, S), flux_aov<E, false>(g, S), Fa);
+#pragma unroll
+		for (int j = 0; j < E::Q; ++j) d[j] = side ? Fa[j] - d[j] : Fa[j];
+	}
+}
+
+// The launch's arguments, or a grid's description, under a pointer of its own:
+// what is read through it is read where it is used, so that a rare path after
+// the row loop keeps no scalars of its own alive through the loop.
+template <typename T>
+__device__ __forceinline__ const T &read_again(const T *p) {
+	using AS4 = const __attribute__((address_space(4))) T *;
+	AS4 q = (AS4)p;
+	asm volatile("" : "+s"(q));
+	return *(const T *)q;
+}
+template <typename R>
+__device__ __forceinline__ const StageArgs<R> &kernel_args_again() {
+	return read_again((const StageArgs<R> *)__builtin_amdgcn_kernarg_segment_ptr());
+}
+
+// Rows y .. y1-1 of a strip's column x (this lane's) in the general form; returns
+// their dt.
+template <typename R, template <typename> class EQ, int DIM, bool PLM, int SLIM>
+__device__ __forceinline__ double general_rows(const StageArgs<R> &a, const GridDesc<R> &g, int x, int y, int y1,
+	double dt)
+{
+	using E = EQ<R>;
+	constexpr int Q = E::Q;
+	const typename E::Par par = E::par(a);
+	const R *src = g.U[a.src];
+	R *out = a.out >= 0 ? g.U[a.out] : g.ping;
+	R *storeD = a.storeD >= 0 ? g.D[a.storeD] : nullptr;
+	const R dt_dx0 = R(dt) / g.dx[0], dt_dx1 = R(dt) / g.dx[1];
+	FastestWave<DIM, E::FASTM> fw;
+	if (x < g.n[0]) {
+		for (; y < y1; ++y) {
+			R d[Q], deriv[Q];
+			face_difference<R, E, 0, PLM, SLIM>(par, a.limiter, g, src, x, y, dt_dx0, d);
+#pragma unroll
+			for (int j = 0; j < Q; ++j) deriv[j] = R(0) - d[j];
+			face_difference<R, E, 1, PLM, SLIM>(par, a.limiter, g, src, x, y, dt_dx1, d);
+#pragma unroll
+			for (int j = 0; j < Q; ++j) deriv[j] = deriv[j] - d[j];
+			Cell<R, E> U;
+			load_plain<R, E>(g, src, (long)y * g.step1 + x, U);
+			finish_cell<R, E, DIM>(a, g, (long)y * g.step1 + x, U, deriv, dt, out, storeD, fw);
+		}
+	}
+	return fw.dt(g.cflScale);
+}
+
 // ------------------------------------------------------- one wave strip
 // Advances the strip (sx, sy) of grid g by one stage: 64 output columns (one
 // per lane; 1D: 60) by rowsPerWave (<= 32) rows. Returns the strip's dt minimum of the new
 // state when the stage reduces dt.
-template <typename R, template <typename> class EQ, int DIM, bool PLM, bool LIM, int FLIM, int SLIM,
-	int RM = ROE_INLINE>
+template <typename R, template <typename> class EQ, int DIM, bool PLM, bool LIM, int FLIM, int SLIM, bool BATCH,
+	int RM>
 __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridDesc<R> &g, int sx, int sy, double dt,
-	int lane, XEdge<R, EQ<R>, PLM, LIM, EDGE_ROWS> *edges, int w, bool share, int yStart = -1)
+	int lane, XEdge<R, EQ<R>, PLM, LIM, EDGE_ROWS> *edges, int w, bool share)
 {
 	using E = EQ<R>;
 	using C = Cell<R, E>;
@@ -831,7 +982,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 	const typename E::Par par = E::par(a);
 	const int lim = PLM ? 0 : a.limiter;   // runtime limiter index when FLIM/SLIM == -1
 	const int slim = a.limiter;
-	FastestWave<DIM> fw;     // of the new state, on the last stage
+	FastestWave<DIM, E::FASTM> fw;     // of the new state, on the last stage
 
 	const int nx = g.n[0];
 	const int ny = DIM >= 2 ? g.n[1] : 1;
@@ -847,8 +998,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 	const R rdt = R(dt);
 	const R dt_dx0 = rdt / g.dx[0];
 	const R dt_dx1 = DIM >= 2 ? rdt / g.dx[1] : R(0);
-	// the strip's rows; the redo kernel starts at the first row it takes over
-	const int y0 = yStart >= 0 ? yStart : sy * g.rowsPerWave;
+	const int y0 = sy * g.rowsPerWave;      // the strip's rows
 	const int y1 = min(sy * g.rowsPerWave + g.rowsPerWave, ny);
 
 	// ---- the strip's edge interfaces for rows y0 .. y1-1: lane j (< 32) the
@@ -937,6 +1087,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 	R dW0[E::NW];           // LIM: dW of interface r-1/2
 	R FaYprev[Q];
 	bool okYprev = true;    // ROE_FLAGGED: interface r-1/2 is regular
+	int yGeneral = y1;      // ROE_FLAGGED: first row left to the general form
 #pragma unroll
 	for (int f = 0; f < C::NV; ++f) { Wm.v[f] = W0.v[f] = W1.v[f] = W2.v[f] = Ry0.v[f] = R(0); }
 #pragma unroll
@@ -1022,13 +1173,10 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 				flux_aov<E, LIM>(g, 0), lane, share ? w * rpw + jr : jr, share ? (w + 1) * rpw + jr : EDGE_ROWS + jr, edge,
 				edgeR, Um, Up, deriv, okX);
 			if constexpr (RM == ROE_FLAGGED) {
-				// an irregular interface of this row: the redo kernel takes the
-				// strip from this row on; nothing of it is stored here
+				// an irregular interface of this row: the strip's rows from
+				// this one on are done below, in the general form
 				if (!wave_all(okYprev && okY && okX)) {
-					if (lane == 0) {
-						const unsigned k = atomicAdd(&g.dev->redoCount, 1u);
-						g.redo[k] = make_int2(sy * g.stripsX + sx, r);
-					}
+					yGeneral = r;
 					break;
 				}
 			}
@@ -1048,57 +1196,8 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 			}
 
 			// ---- integrator combine (rk.lua:155-174, fe.lua:50), constrainU
-			if (outLane) {
-				long off = (long)r * g.step1 + x;
-				double acc[Q];
-#pragma unroll
-				for (int j = 0; j < Q; ++j) acc[j] = 0.;
-				for (int k = 0; k < a.nAlpha; ++k) {
-					const bool fromSrc = a.accU[k] == a.src;
-					const R *Uk = g.U[a.accU[k]];
-					double al = a.alpha[k];
-#pragma unroll
-					for (int j = 0; j < Q; ++j) {
-						if (!E::active(j)) continue;
-						R u = fromSrc ? U.v[j] : Uk[j * g.ps + off];
-						acc[j] = acc[j] + (double)u * al;
-					}
-				}
-				for (int k = 0; k < a.nStoredD; ++k) {
-					const R *Dk = g.D[a.accD[k]];
-					double c = (double)R(a.beta[k] * dt);
-#pragma unroll
-					for (int j = 0; j < Q; ++j)
-						if (E::active(j)) acc[j] = acc[j] + (double)Dk[j * g.ps + off] * c;
-				}
-				if (storeD) {
-#pragma unroll
-					for (int j = 0; j < Q; ++j)
-						if (E::active(j)) storeD[j * g.ps + off] = deriv[j];
-				}
-				if (a.betaNew != 0.) {
-					double c = (double)R(a.betaNew * dt);
-#pragma unroll
-					for (int j = 0; j < Q; ++j)
-						if (E::active(j)) acc[j] = acc[j] + (double)deriv[j] * c;
-				}
-				E::constrain(a.pd, acc);
-				R o[Q];
-#pragma unroll
-				for (int j = 0; j < Q; ++j) {
-					o[j] = R(acc[j]);
-					if (E::active(j)) out[j * g.ps + off] = o[j];
-				}
-				if (a.reduceSlot >= 0) {
-					double ud[C::NV];
-#pragma unroll
-					for (int j = 0; j < Q; ++j) ud[j] = (double)o[j];
-#pragma unroll
-					for (int j = Q; j < C::NV; ++j) ud[j] = (double)U.v[j];
-					E::template fastest<DIM>(a.pd, ud, fw.lam);
-					fw.seen = true;
-				}
-			}
+			if (outLane)
+				finish_cell<R, E, DIM>(a, g, (long)r * g.step1 + x, U, deriv, dt, out, storeD, fw);
 		}
 
 		// ---- advance the row window
@@ -1110,7 +1209,15 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 		}
 	}
 	}
-	return a.reduceSlot >= 0 ? fw.dt(g.dxD) : INFINITY;
+	if constexpr (RM == ROE_FLAGGED) {
+		if (yGeneral < y1) {
+			const StageArgs<R> &aa = kernel_args_again<R>();
+			const double d = general_rows<R, EQ, DIM, PLM, SLIM>(aa, BATCH ? read_again(&g) : aa.g, x, yGeneral, y1,
+				dt);
+			return a.reduceSlot >= 0 ? fmin(d, fw.dt(g.cflScale)) : INFINITY;
+		}
+	}
+	return a.reduceSlot >= 0 ? fw.dt(g.cflScale) : INFINITY;
 }
 
 // dt of this step for grid g (solverbase.lua:3016): cfl * min, or a host value
@@ -1143,21 +1250,20 @@ __device__ __forceinline__ void stage_reduce(const StageArgs<R> &a, const GridDe
 // ---------------------------------------------------------- the kernels
 // Plain form: one grid, one wave per strip. The 2D FAST kernels of the Euler
 // equations with the Roe flux and no flux limiter take the collected Roe form
-// only (ROE_FLAGGED) and leave any strip with an irregular interface, from
-// that row on, to stage_kernel_redo, launched after them on the same stream.
+// in their row loop (ROE_FLAGGED).
 // The FP64 form of 'plm cons' or no reconstruction without an out-of-plane
 // velocity needs about 128 registers, the most that lets a SIMD hold four
 // waves: it is held to that (the allocator takes 130 on its own, three waves).
 template <typename R, class E, int DIM>
 __host__ __device__ constexpr int plain_min_blocks(bool lim) {
-	return sizeof(R) == 8 && redo_form<E, DIM>(lim) && !E::active(3) && !E::PLM_PRIM && !E::PLM_EIG && !E::PLM_CONS_FLUX
+	return sizeof(R) == 8 && flagged_form<E, DIM>(lim) && !E::active(3) && !E::PLM_PRIM && !E::PLM_EIG && !E::PLM_CONS_FLUX
 		&& !E::PLM_ATHENA && !E::PLM_PPM && !E::PLM_EIG_PRIM && !E::PLM_EIG_PRIM_REF ? 4 : 1;
 }
 
 template <typename R, template <typename> class EQ, int DIM, bool PLM, bool LIM, int FLIM, int SLIM>
 __global__ void __launch_bounds__(256, (plain_min_blocks<R, EQ<R>, DIM>(LIM))) stage_kernel(const StageArgs<R> a)
 {
-	constexpr int RM = redo_form<EQ<R>, DIM>(LIM) ? ROE_FLAGGED : ROE_INLINE;
+	constexpr int RM = flagged_form<EQ<R>, DIM>(LIM) ? ROE_FLAGGED : ROE_INLINE;
 	const int lane = threadIdx.x & 63;
 	int blk = a.xcdRemap ? xcd_block(blockIdx.x, a.nBlocks) : (int)blockIdx.x;
 	const int waveInBlock = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1173,64 +1279,9 @@ __global__ void __launch_bounds__(256, (plain_min_blocks<R, EQ<R>, DIM>(LIM))) s
 	// band (the host sets the flag only where the strips per row are a
 	// multiple of 4, so every block is whole)
 	const bool share = DIM == 2 && strip_edges(DIM, EQ<R>::SOURCE) && a.shareEdges != 0 && blockDim.x == 256;
-	double dtLocal = stage_strip<R, EQ, DIM, PLM, LIM, FLIM, SLIM, RM>(a, g, sx, sy, dt, lane, edges, waveInBlock,
+	double dtLocal = stage_strip<R, EQ, DIM, PLM, LIM, FLIM, SLIM, false, RM>(a, g, sx, sy, dt, lane, edges, waveInBlock,
 		share);
 	stage_reduce(a, g, dtLocal, item, lane);
-}
-
-// The strips a stage kernel left (from their first irregular row on), with
-// the Roe form chosen per interface (ROE_INLINE): the entries of every grid's
-// redo list (one grid for the plain form, a.grids for the batched one) are
-// numbered one after the other, and wave k takes entries k, k + W, k + 2W, ...
-// (W = waves launched). The rows it takes were not written by the stage
-// kernel, so their inputs are as the stage began; their dt joins the same
-// slot. The lists' lengths are read 64 grids at a time, one per lane; when
-// every list is empty (the usual case) the kernel ends there, with nothing to
-// clear. Otherwise the last block to finish empties the lists for the next
-// stage (every wave has read the lengths by then); no wave depends on another.
-template <typename R, template <typename> class EQ, int DIM, bool PLM, bool LIM, int FLIM, int SLIM>
-__global__ void __launch_bounds__(256) stage_kernel_redo(const StageArgs<R> a)
-{
-	const int lane = threadIdx.x & 63;
-	const int waveInBlock = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-	const long wave = (long)blockIdx.x * (blockDim.x >> 6) + waveInBlock;
-	const long nWaves = (long)gridDim.x * (blockDim.x >> 6);
-	__shared__ XEdge<R, EQ<R>, PLM, LIM, EDGE_ROWS> edges[4];
-	__shared__ unsigned lastBlock;
-	const bool batched = a.grids != nullptr;
-	const int nGrids = batched ? a.nGrids : 1;
-	long base = 0;     // entries of the grids before the current one
-	for (int g0 = 0; g0 < nGrids; g0 += 64) {
-		const int gi = g0 + lane;
-		unsigned c = 0u;
-		if (gi < nGrids) c = (batched ? a.grids[gi].dev : a.g.dev)->redoCount;
-		unsigned long long pending = __ballot(c != 0u);
-		while (pending) {
-			const int j = __ffsll((long long)pending) - 1;
-			pending &= pending - 1;
-			const long n = (long)__shfl(c, j);
-			const GridDesc<R> &g = batched ? a.grids[g0 + j] : a.g;
-			const double dt = stage_dt(a, g);
-			// this wave's first entry at or after base
-			for (long k = base + ((wave - base) % nWaves + nWaves) % nWaves; k < base + n; k += nWaves) {
-				const int2 e = g.redo[k - base];
-				const int sx = e.x % g.stripsX, sy = e.x / g.stripsX;
-				double dtLocal = stage_strip<R, EQ, DIM, PLM, LIM, FLIM, SLIM, ROE_INLINE>(a, g, sx, sy, dt, lane,
-					edges, waveInBlock, false, e.y);
-				stage_reduce(a, g, dtLocal, e.x, lane);
-			}
-			base += n;
-		}
-	}
-	if (base == 0) return;     // the same for every wave of the launch
-	DevScalars *d = batched ? a.grids[0].dev : a.g.dev;
-	__syncthreads();
-	if (threadIdx.x == 0) lastBlock = atomicAdd(&d->redoDone, 1u) == gridDim.x - 1 ? 1u : 0u;
-	__syncthreads();
-	if (lastBlock && threadIdx.x < 64) {
-		for (int gi = lane; gi < nGrids; gi += 64) (batched ? a.grids[gi].dev : a.g.dev)->redoCount = 0u;
-		if (lane == 0) d->redoDone = 0u;
-	}
 }
 
 // Dynamic LDS of the batched kernel: the strip-edge slices of its waves
@@ -1241,12 +1292,11 @@ extern __shared__ __align__(16) unsigned char batch_lds[];
 // the batch; wave k takes items k, k + W, k + 2W, ... (W = waves launched).
 // Items are numbered grid by grid (GridDesc::itemBase), so the owning grid of
 // an item is found by a wave-uniform binary search. The Roe form is the plain
-// kernel's (ROE_FLAGGED where it applies, with the same redo kernel after it),
-// so a grid advances to the same bits batched or alone.
+// kernel's, so a grid advances to the same bits batched or alone.
 template <typename R, template <typename> class EQ, int DIM, bool PLM, bool LIM, int FLIM, int SLIM>
 __global__ void __launch_bounds__(256) stage_kernel_batch(const StageArgs<R> a)
 {
-	constexpr int RM = redo_form<EQ<R>, DIM>(LIM) ? ROE_FLAGGED : ROE_INLINE;
+	constexpr int RM = flagged_form<EQ<R>, DIM>(LIM) ? ROE_FLAGGED : ROE_INLINE;
 	const int lane = threadIdx.x & 63;
 	int blk = a.xcdRemap ? xcd_block(blockIdx.x, a.nBlocks) : (int)blockIdx.x;
 	const int waveInBlock = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1270,7 +1320,7 @@ __global__ void __launch_bounds__(256) stage_kernel_batch(const StageArgs<R> a)
 		const int sx = (int)(local % g.stripsX);
 		const int sy = (int)(local / g.stripsX);
 		if (local == 0) stage_first_strip(a, g, dt, lane);
-		double dtLocal = stage_strip<R, EQ, DIM, PLM, LIM, FLIM, SLIM, RM>(a, g, sx, sy, dt, lane, edges, waveInBlock,
+		double dtLocal = stage_strip<R, EQ, DIM, PLM, LIM, FLIM, SLIM, true, RM>(a, g, sx, sy, dt, lane, edges, waveInBlock,
 			false);
 		stage_reduce(a, g, dtLocal, local, lane);
 	}

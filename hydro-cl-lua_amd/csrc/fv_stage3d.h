@@ -99,7 +99,7 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 	const typename E::Par par = E::par(a);
 	const int lim = PLM ? 0 : a.limiter;
 	const int slim = a.limiter;
-	FastestWave<3> fw;     // of the new state, on the last stage
+	FastestWave<3, E::FASTM> fw;     // of the new state, on the last stage
 
 	const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
 	const R *src = g.U[a.src];
@@ -286,57 +286,8 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 			}
 
 			// ---- integrator combine, constrainU, new state's dt
-			if (outLane) {
-				long off = ((long)r * ny + y) * g.step1 + x;
-				double acc[Q];
-#pragma unroll
-				for (int j = 0; j < Q; ++j) acc[j] = 0.;
-				for (int k = 0; k < a.nAlpha; ++k) {
-					const bool fromSrc = a.accU[k] == a.src;
-					const R *Uk = g.U[a.accU[k]];
-					double al = a.alpha[k];
-#pragma unroll
-					for (int j = 0; j < Q; ++j) {
-						if (!E::active(j)) continue;
-						R u = fromSrc ? U.v[j] : Uk[j * g.ps + off];
-						acc[j] = acc[j] + (double)u * al;
-					}
-				}
-				for (int k = 0; k < a.nStoredD; ++k) {
-					const R *Dk = g.D[a.accD[k]];
-					double c = (double)R(a.beta[k] * dt);
-#pragma unroll
-					for (int j = 0; j < Q; ++j)
-						if (E::active(j)) acc[j] = acc[j] + (double)Dk[j * g.ps + off] * c;
-				}
-				if (storeD) {
-#pragma unroll
-					for (int j = 0; j < Q; ++j)
-						if (E::active(j)) storeD[j * g.ps + off] = deriv[j];
-				}
-				if (a.betaNew != 0.) {
-					double c = (double)R(a.betaNew * dt);
-#pragma unroll
-					for (int j = 0; j < Q; ++j)
-						if (E::active(j)) acc[j] = acc[j] + (double)deriv[j] * c;
-				}
-				E::constrain(a.pd, acc);
-				R o[Q];
-#pragma unroll
-				for (int j = 0; j < Q; ++j) {
-					o[j] = R(acc[j]);
-					if (E::active(j)) out[j * g.ps + off] = o[j];
-				}
-				if (a.reduceSlot >= 0) {
-					double ud[NV];
-#pragma unroll
-					for (int j = 0; j < Q; ++j) ud[j] = (double)o[j];
-#pragma unroll
-					for (int j = Q; j < NV; ++j) ud[j] = (double)U.v[j];
-					E::template fastest<3>(a.pd, ud, fw.lam);
-					fw.seen = true;
-				}
-			}
+			if (outLane)
+				finish_cell<R, E, 3>(a, g, ((long)r * ny + y) * g.step1 + x, U, deriv, dt, out, storeD, fw);
 		}
 
 		// ---- advance the plane window
@@ -344,7 +295,7 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 		else { W0 = W1; }
 	}
 	}
-	return a.reduceSlot >= 0 ? fw.dt(g.dxD) : INFINITY;
+	return a.reduceSlot >= 0 ? fw.dt(g.cflScale) : INFINITY;
 }
 
 // The halo wave of the block: per output plane, the rows y0-2, y0-1 and
@@ -378,13 +329,16 @@ __device__ __forceinline__ void stage_halo3d(const StageArgs<R> &a, const GridDe
 	const int rowOf[4] = {y0 - 2, y0 - 1, y0 + W, y0 + W + 1};
 	const int slotOf[4] = {0, 1, W + 2, W + 3};
 	C h[4];
+	const bool xPlain = wave_all(mx.fixedFace < 0 && !mx.mirror);
 	auto loadHalo = [&](int zz) {
 		const Mapped mz = map_coord(zz, nz, g.bc[4], g.bc[5], 4);
 #pragma unroll
 		for (int k = 0; k < 4; ++k) {
 			if (!TWO && (k == 0 || k == 3)) continue;
 			const Mapped my = map_coord(rowOf[k], ny, g.bc[2], g.bc[3], 2);
-			load_cell3<R, E>(g, src, mx, my, mz, h[k]);
+			if (xPlain && my.fixedFace < 0 && !my.mirror && mz.fixedFace < 0 && !mz.mirror)
+				load_plain<R, E>(g, src, ((long)mz.idx * g.n[1] + my.idx) * g.step1 + mx.idx, h[k]);
+			else load_cell3<R, E>(g, src, mx, my, mz, h[k]);
 		}
 	};
 	if (z0 < z1) loadHalo(z0);

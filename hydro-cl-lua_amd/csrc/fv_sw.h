@@ -260,7 +260,7 @@ struct Eqn {
 				C_nLen = 0.;
 				v_n = 0.;
 			}
-			lam[s] = fmax(lam[s], fabs(v_n) + C_nLen);
+			lam[s] = fabs(v_n) + C_nLen;
 		}
 	}
 

@@ -168,19 +168,10 @@ static int solver_stage(hydro_solver *h, int s, int useSlot, double hostDt, int 
 	// edge columns they need (5 rows-per-wave interfaces in one wave)
 	a.shareEdges = g.dim == 2 && strip_edges(2, eqn_has_source(g.cfg.eqn)) && a.g.stripsX % 4 == 0 &&
 		5 * a.g.rowsPerWave <= WAVE;
-	const bool redo = redo_kernels(g.cfg);
 	if (ev0) HIPCHECK(hipEventRecord(ev0, h->stream));
 	const StageKey k = stage_key(g);
 	hipError_t e = launch_stage<R>(k, a, dim3(a.nBlocks), dim3(256), h->stream);
 	if (e != hipSuccess) return fail("stage kernel launch: %s", hipGetErrorString(e));
-	if (redo) {
-		// the strips the stage kernel left to the general Roe form (usually none)
-		a.redoPass = 1;
-		a.shareEdges = 0;
-		a.nBlocks = REDO_BLOCKS;
-		e = launch_stage<R>(k, a, dim3(REDO_BLOCKS), dim3(256), h->stream);
-		if (e != hipSuccess) return fail("redo kernel launch: %s", hipGetErrorString(e));
-	}
 	if (ev1) HIPCHECK(hipEventRecord(ev1, h->stream));
 	return 0;
 }
