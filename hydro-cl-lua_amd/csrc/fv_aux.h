@@ -58,7 +58,7 @@ template <typename R, template <typename> class EQ, int DIM>
 __global__ void __launch_bounds__(256) dt_kernel(const GridArgs<R> g) {
 	using E = EQ<R>;
 	constexpr int Q = E::Q;
-	FastestWave<DIM, E::FASTM> fw;
+	FastestOf<R, E, DIM> fw;
 	for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < g.ncell; c += (long)gridDim.x * blockDim.x) {
 		double u[Q + E::NSTAT];
 #pragma unroll

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include "../../include/hydro_hip.h"
+#include "fv_math.h"
 
 namespace hydro {
 
@@ -28,6 +29,14 @@ __host__ __device__ constexpr bool strip_edges(int dim, bool source) { return di
 constexpr int EDGE_ROWS = WAVE / 2;// rows per wave item at most (2D): the strip-edge
                                    // interfaces of each row take a lane per side
 constexpr int EDGE_PLANES = 16;    // planes per block chunk at most (3D)
+
+// 2D tile kernel (fv_tile.h): a block is TILE_W row waves, a row each, and one
+// halo wave. Its strips have 64 columns, with edge interfaces from the halo wave;
+// with a flux limiter an edge takes three interface preparations, twice a row's:
+// there, as with a source term, the strip loads a halo and outputs 60.
+constexpr int TILE_W = 3;
+constexpr int TILE_WAVES = TILE_W + 1;
+__host__ __device__ constexpr bool tile_edges(bool source, bool lim) { return !source && !lim; }
 
 // 3D stage kernel: a block is W row waves (rows of a strip that share one
 // plane through LDS) and one halo wave that loads the rows outside the block
@@ -130,6 +139,7 @@ struct StageArgs {
 	int resetSlot;            // slot to clear to +inf, -1 none
 	int reduceSlot;           // slot to min-reduce the new state's dt into, -1 none
 	int advanceTime;          // t += dt, dt stored
+	int tile;                 // plain 2D launch of the tile kernel (fv_tile.h)
 	int shareEdges;           // plain 2D launch: one strip-edge pass per block of 4 x-adjacent strips
 	int stepInTick;           // batch: skip grids with stepsLeft <= stepInTick
 	// equation parameters in the stencil type and in double (for the FP64
@@ -276,15 +286,14 @@ __device__ __forceinline__ void atomic_min_pos(double *p, double v) {
 }
 
 // The CFL step of the cells a lane has seen (calcDT.cl:38-73: the minimum of
-// dx / max(1e-9, |lambda|) over cells and axes) from the fastest wave: division
-// is monotonic, so dx / max is the minimum, with one division per wave in place
-// of one per axis and cell. The EXACT kernels keep the fastest wave of each
-// axis, whose dx / max is the reference's minimum bit for bit; the FAST ones
-// keep one value, every axis' waves scaled to the first axis' cell length (an
-// exact 1 where the lengths are equal): two registers less through the row loop.
-template <int DIM, bool FAST>
+// dx / max(1e-9, |lambda|) over cells and axes) from the fastest wave of each
+// axis: division is monotonic, so dx / max is the minimum, with one division per
+// axis and wave in place of one per axis and cell. ONE (the FP64 FAST kernels):
+// one value, every axis' waves scaled to the first axis' cell length (an exact 1
+// where the lengths are equal), two registers less through the row loop.
+template <int DIM, bool FAST, bool ONE>
 struct FastestWave {
-	static constexpr int N = FAST ? 1 : DIM;
+	static constexpr int N = ONE ? 1 : DIM;
 	double lam[N];
 	bool seen;
 	__device__ __forceinline__ FastestWave() : seen(false) {
@@ -295,23 +304,26 @@ struct FastestWave {
 	__device__ __forceinline__ void add(const CflScale &c, const double *l) {
 #pragma unroll
 		for (int s = 0; s < DIM; ++s) {
-			if constexpr (FAST) lam[0] = fmax(lam[0], fmax(1e-9, l[s]) * c.scale[s]);
+			if constexpr (ONE) lam[0] = fmax(lam[0], fmax(1e-9, l[s]) * c.scale[s]);
 			else lam[s] = fmax(lam[s], l[s]);
 		}
 		seen = true;
 	}
 	__device__ __forceinline__ double dt(const CflScale &c) const {
+		using MD = Math<double, FAST>;
 		double d = INFINITY;
-		if constexpr (FAST) {
-			d = c.len / lam[0];
+		if constexpr (ONE) {
+			d = MD::div(c.len, lam[0]);
 		} else {
 #pragma unroll
 			for (int s = 0; s < DIM; ++s)
-				if (c.dx[s] > 0.) d = fmin(d, c.dx[s] / fmax(1e-9, lam[s]));
+				if (c.dx[s] > 0.) d = fmin(d, MD::div(c.dx[s], fmax(1e-9, lam[s])));
 		}
 		return seen ? d : INFINITY;
 	}
 };
+template <typename R, class E, int DIM>
+using FastestOf = FastestWave<DIM, E::FASTM, E::FASTM && sizeof(R) == 8>;
 
 // Logical block id with blocks spread so that each XCD (blocks are dealt
 // round-robin over the 8 XCDs) gets a contiguous range of logical ids, so

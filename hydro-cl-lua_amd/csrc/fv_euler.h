@@ -395,6 +395,52 @@ struct EulerT {
 			return p.g1 * t;
 		}
 
+		// Twice the Roe flux of a regular interface as the sum over the waves of
+		// |lambda| (l . dU) r, with R's columns collected.
+		template <int S>
+		__device__ static __forceinline__ void roe_sum_waves(const RoeState &q, const R *UL, const R *UR, const R *X,
+			R dp, R dn, R *F) {
+			constexpr int A = S, B = (S + 1) % 3, C = (S + 2) % 3;
+			const R c = q.c, vn = q.v[A];
+			const R cB = c * dn;
+			const R ic2 = q.ic * q.ic, hic2 = R(.5) * ic2;
+			// L dU
+			R y[5];
+			y[0] = (dp + cB) * hic2;
+			y[4] = (dp - cB) * hic2;
+			y[1] = X[0] - dp * ic2;
+			y[2] = B < NVEL ? X[1 + B] - q.v[B] * X[0] : R(0);
+			y[3] = C < NVEL ? X[1 + C] - q.v[C] * X[0] : R(0);
+			// |Lambda| L dU
+			const R an = fabs(vn);
+			const R f0 = fabs(vn - c) * y[0], f4 = fabs(vn + c) * y[4];
+			const R f1 = an * y[1], fB = an * y[2], fC = an * y[3];
+			// R (|Lambda| L dU)
+			const R z0 = f0 + f1 + f4;
+			const R d40 = f4 - f0;
+			R zm[3];
+			zm[A] = vn * z0 + c * d40;
+			zm[B] = B < NVEL ? q.v[B] * z0 + fB : R(0);
+			zm[C] = C < NVEL ? q.v[C] * z0 + fC : R(0);
+			R z4 = q.H * (f0 + f4) + (c * vn) * d40 + q.hq * f1;
+			if constexpr (B < NVEL) z4 = z4 + q.v[B] * fB;
+			if constexpr (C < NVEL) z4 = z4 + q.v[C] * fC;
+			// F(UL) + F(UR) - z
+			const R vnL = q.vL[A], vnR = q.vR[A];
+			F[0] = (UL[1 + A] + UR[1 + A]) - z0;
+#pragma unroll
+			for (int i = 0; i < 3; ++i) {
+				if (i < NVEL || i == A) {
+					R fs = UL[1 + i] * vnL + UR[1 + i] * vnR;
+					if (i == A) fs = fs + (q.PL + q.PR);
+					F[1 + i] = fs - zm[i];
+				} else {
+					F[1 + i] = R(0);
+				}
+			}
+			F[4] = (q.EPL * vnL + q.EPR * vnR) - z4;
+		}
+
 		// Twice the Roe flux, F(UL) + F(UR) - R |Lambda| L (UR - UL) (roe.cl:17-163
 		// without a flux limiter; the caller folds the half into the flux's area
 		// factor, which is exact), of a regular interface, from roe_state. With an = |vn|, e = max(an, c) - an and D = vn limited to
@@ -406,8 +452,8 @@ struct EulerT {
 		// average makes dE = dp / g1 + v.dm - v^2/2 drho exact): about 20 fewer
 		// instructions per interface than R |Lambda| L dU wave by wave, and 0.35-
 		// 0.9 of its rounding error (FP32 against FP64 on random states, Mach .05
-		// to 3). The stage kernels are bound by VALU issue and latency: 2D FP32
-		// 1024^2 24.8 -> 23.8 us per stage, 3D 'plm cons' 128^3 68.2 -> 65.0 us.
+		// to 3). FP64 only: FP32 flows carry a change of rounding to their seventh
+		// digit, the time step's among them, and keep the sum over the waves.
 		// Returns whether this lane's interface is regular (F holds the result
 		// only then).
 		template <int S>
@@ -421,6 +467,10 @@ struct EulerT {
 			const R dp = roe_dp(p, q, X);
 			const R dn = vn * X[0] - X[1 + A];
 			const R an = fabs(vn);
+			if constexpr (sizeof(R) == 4) {
+				roe_sum_waves<S>(q, UL, UR, X, dp, dn, F);
+				return q.ok;
+			}
 			const R e = fmax(c - an, R(0));
 			const R Dc = fmax(fmin(vn, c), -c) * ic;
 			const R a1 = (dp * ic) * (e * ic) - dn * Dc;
@@ -503,17 +553,19 @@ struct EulerT {
 			l[4] = vn + e.Cs;
 		}
 
-		// constrainU (euler.cl:697-717) on a state in double. FAST: a state whose
+		// constrainU (euler.cl:697-717) on a state in double. FAST FP64: a state whose
 		// density is at least rhoMin and whose internal energy, rho e = E -
 		// m^2 / (2 rho), is clear of PMin's is left as it is (the reference's
 		// cons -> prim -> cons round trip changes it by roundings only); the
 		// others, and NaNs, take the whole form. The test times rho needs no
 		// division: 5 instructions for the usual cell in place of 26 (with the
-		// CFL step's division taken once per wave, FastestWave: 2D FP32 2048^2
-		// 64.1 -> 60.4 us per stage, 3D FP32 256^3 598 -> 581 us; the error of
-		// KH FP64 runs against 64-bit references falls by 40%).
+		// CFL step's division taken once per wave, FastestWave: KH 1024^2 FP64
+		// 34.1 -> 32.0 us per stage, and 40% less error of such runs against
+		// 64-bit references). FP32 keeps the round trip: it changes the rounding
+		// to FP32 of one value in 1e9, and an FP32 flow carries that to its
+		// seventh digit within some hundred steps, the time step's among them.
 		__device__ static __forceinline__ void constrain(const EqnParD &pd, double *U) {
-			if constexpr (FAST) {
+			if constexpr (FAST && sizeof(R) == 8) {
 				const double rhoEInt = U[0] * U[4] - .5 * lenSq3(U + 1);
 				const bool clear = U[0] >= pd.rhoMin && rhoEInt > U[0] * pd.eIntSafe;
 				if (!wave_all(clear)) {

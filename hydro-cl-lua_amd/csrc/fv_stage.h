@@ -823,7 +823,7 @@ __device__ __forceinline__ void strip_x(const typename E::Par &par, int lim, int
 // constrainU, the store, and the new state's fastest waves on the last stage.
 template <typename R, class E, int DIM>
 __device__ __forceinline__ void finish_cell(const StageArgs<R> &a, const GridDesc<R> &g, long off, const Cell<R, E> &U,
-	const R *deriv, double dt, R *out, R *storeD, FastestWave<DIM, E::FASTM> &fw)
+	const R *deriv, double dt, R *out, R *storeD, FastestOf<R, E, DIM> &fw)
 {
 	constexpr int Q = E::Q;
 	double acc[Q];
@@ -949,7 +949,7 @@ __device__ __forceinline__ double general_rows(const StageArgs<R> &a, const Grid
 	R *out = a.out >= 0 ? g.U[a.out] : g.ping;
 	R *storeD = a.storeD >= 0 ? g.D[a.storeD] : nullptr;
 	const R dt_dx0 = R(dt) / g.dx[0], dt_dx1 = R(dt) / g.dx[1];
-	FastestWave<DIM, E::FASTM> fw;
+	FastestOf<R, E, DIM> fw;
 	if (x < g.n[0]) {
 		for (; y < y1; ++y) {
 			R d[Q], deriv[Q];
@@ -982,7 +982,7 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 	const typename E::Par par = E::par(a);
 	const int lim = PLM ? 0 : a.limiter;   // runtime limiter index when FLIM/SLIM == -1
 	const int slim = a.limiter;
-	FastestWave<DIM, E::FASTM> fw;     // of the new state, on the last stage
+	FastestOf<R, E, DIM> fw;     // of the new state, on the last stage
 
 	const int nx = g.n[0];
 	const int ny = DIM >= 2 ? g.n[1] : 1;

@@ -99,7 +99,7 @@ __device__ __forceinline__ double stage_rows3d(const StageArgs<R> &a, const Grid
 	const typename E::Par par = E::par(a);
 	const int lim = PLM ? 0 : a.limiter;
 	const int slim = a.limiter;
-	FastestWave<3, E::FASTM> fw;     // of the new state, on the last stage
+	FastestOf<R, E, 3> fw;     // of the new state, on the last stage
 
 	const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
 	const R *src = g.U[a.src];
