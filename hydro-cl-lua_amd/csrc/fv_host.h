@@ -172,6 +172,7 @@ struct Grid {
 	int slot;           // dt slot of the next step
 	int dtValid;        // slot holds the min for the current state
 	int rowsPerWave;
+	int tile;           // plain 2D solver: the tile kernel in place of the marching one
 	int nvel;           // Euler: velocity components that are not identically zero
 	std::vector<double> ePot;   // Euler ePot of the last upload (dynamics-neutral)
 };
@@ -305,6 +306,32 @@ static int default_rows(const hydro_cfg &cfg, int nx, int ny, int nz) {
 	return best;
 }
 
+// The tile kernel's strips (its blocks per TILE_W rows) and blocks on a 2D grid.
+static int tile_strips(const hydro_cfg &cfg) {
+	const bool lim = cfg.plm == HYDRO_PLM_NONE && cfg.flux == HYDRO_FLUX_ROE && cfg.flux_limiter != HYDRO_LIMITER_DONOR_CELL;
+	const int so = strip_out(tile_edges(eqn_has_source(cfg.eqn), lim));
+	return (cfg.size[0] + so - 1) / so;
+}
+static long tile_blocks(const hydro_cfg &cfg) {
+	return (long)tile_strips(cfg) * ((cfg.size[1] + TILE_W - 1) / TILE_W);
+}
+
+// Whether the plain 2D solver takes the tile kernel (fv_tile.h) and not the
+// marching one. Its time is about 5.2 us plus 1.4-1.8 us (IEEE 3) for each block
+// a CU has to run; the marching kernel's is flat (FAST 10-27 us, IEEE 22-35 us, by
+// the scheme) while its waves are all resident at once and then grows at half to
+// two thirds of that rate. Measured at 4 blocks per CU (384^2), tile / marching:
+// 'plm cons' FP64 10.4 / 13.8, FP32 8.9 / 11.5, flux-limited 11.6 / 15.7, shallow
+// water 11.4 / 13.9, GLM-Maxwell FP32 10.2 / 12.2, FP64 14.2 / 14.3, HLLC 11.7 /
+// 17.1, 'plm athena' 18.3 / 27.1 us; 'plm cons' at 5.3 (512^2) 15.0 / 14.8. IEEE at
+// 14 (about 830^2): 47.1 / 50.9 at 800^2.
+static bool tile_form(const hydro_cfg &cfg) {
+	if (cfg.dim != 2) return false;
+	const bool heavy = cfg.eqn == HYDRO_EQN_GLM_MAXWELL && cfg.precision == HYDRO_REAL_F64;
+	const double perCU = !cfg.fast_math ? 14. : heavy ? 4. : 4.5;
+	return (double)tile_blocks(cfg) <= perCU * (double)device_cus();
+}
+
 static void grid_init(Grid &g, const hydro_cfg &cfg) {
 	g.cfg = cfg;
 	g.dim = cfg.dim;
@@ -327,6 +354,7 @@ static void grid_init(Grid &g, const hydro_cfg &cfg) {
 	g.dtValid = 0;
 	g.nvel = 3;
 	g.rowsPerWave = default_rows(cfg, g.n[0], g.n[1], g.n[2]);
+	g.tile = tile_form(cfg);
 }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -496,6 +524,7 @@ static void stage_args(const Grid &g, int s, StageArgs<R> &a) {
 	a.advanceTime = 0;
 	a.xcdRemap = 1;
 	a.shareEdges = 0;
+	a.tile = 0;
 }
 
 static StageKey stage_key_cfg(const hydro_cfg &cfg, int nvel) {

@@ -43,9 +43,10 @@ template <typename R> struct GridArgs;
 template <typename R>
 hipError_t launch_stage(const StageKey &k, const StageArgs<R> &a, dim3 grid, dim3 block, hipStream_t s);
 extern thread_local int stage_occupancy;
-// the same for one math policy and dimension (launch_stage picks by k.fast and
-// k.dim); each is defined in a translation unit of its own
-template <typename R, bool FAST, int DIM>
+// The same for one math policy, dimension and form (launch_stage picks by k.fast,
+// k.dim and the launch); each is defined in a translation unit of its own.
+enum { FORM_PLAIN = 0, FORM_TILE = 1, FORM_BATCH = 2 };
+template <typename R, bool FAST, int DIM, int FORM>
 hipError_t launch_stage_dim(const StageKey &k, const StageArgs<R> &a, dim3 grid, dim3 block, hipStream_t s);
 
 template <typename R>

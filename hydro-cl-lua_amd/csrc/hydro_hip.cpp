@@ -113,14 +113,17 @@ extern "C" int hydro_set_launch(hydro_solver *h, int rows_per_wave, int xcd_rema
 	const int maxRows = h->g.dim == 3 ? EDGE_PLANES : EDGE_ROWS;
 	if (rows_per_wave < 0 || rows_per_wave > maxRows)
 		return fail("rows_per_wave %d out of range 0..%d", rows_per_wave, maxRows);
-	if (rows_per_wave > 0 && h->g.dim >= 2) h->g.rowsPerWave = rows_per_wave;
+	if (rows_per_wave > 0 && h->g.dim >= 2) {
+		h->g.rowsPerWave = rows_per_wave;
+		h->g.tile = 0;       // the caller's rows: the marching kernel
+	}
 	if (xcd_remap > 0) h->xcdRemap = xcd_remap == 1;
 	return 0;
 }
 
 extern "C" int hydro_get_launch(const hydro_solver *h, int *rows_per_wave, int *xcd_remap) {
 	if (!h) return fail("NULL handle");
-	if (rows_per_wave) *rows_per_wave = h->g.rowsPerWave;
+	if (rows_per_wave) *rows_per_wave = h->g.tile ? 1 : h->g.rowsPerWave;
 	if (xcd_remap) *xcd_remap = h->xcdRemap ? 1 : 2;
 	return 0;
 }
@@ -168,6 +171,11 @@ static int solver_stage(hydro_solver *h, int s, int useSlot, double hostDt, int 
 	// edge columns they need (5 rows-per-wave interfaces in one wave)
 	a.shareEdges = g.dim == 2 && strip_edges(2, eqn_has_source(g.cfg.eqn)) && a.g.stripsX % 4 == 0 &&
 		5 * a.g.rowsPerWave <= WAVE;
+	if (g.tile) {
+		a.tile = 1;
+		a.g.stripsX = tile_strips(g.cfg);
+		a.nBlocks = (int)tile_blocks(g.cfg);
+	}
 	if (ev0) HIPCHECK(hipEventRecord(ev0, h->stream));
 	const StageKey k = stage_key(g);
 	hipError_t e = launch_stage<R>(k, a, dim3(a.nBlocks), dim3(256), h->stream);
