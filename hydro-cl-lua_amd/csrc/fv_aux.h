@@ -52,6 +52,123 @@ __global__ void __launch_bounds__(256) nonfinite_kernel(const R *U, const R *sta
 	if (wave_any(bad) && (threadIdx.x & 63) == 0) atomicOr(flag, 1u);
 }
 
+// ------------------------------------------------------------ host transfers
+// The reference's ghosted cons_t buffer (cells of S reals, x fastest) against the
+// planes of the interior, one pinned chunk of consecutive cells at a time. The
+// chunk lives in host memory that the kernel addresses directly, so the bus is
+// crossed once, in 16-byte pieces of consecutive lanes; the transpose between
+// cells and planes goes through LDS. Bound by the bus (about 50 GB/s; 3.2 MB of a
+// 256^2 FP64 state in 70 us).
+template <typename R>
+struct CellBuffer {
+	R *U;                 // q integrated planes
+	R *stat;              // static planes
+	long ps;
+	int n[3], dim;
+	int q, nstat, S;      // planes, and reals per cell of the buffer
+	int bc[6];
+	R fixedv[6][HYDRO_MAX_STATES];
+	int vec1, vec2;       // first fields of the vectors a mirror reflects (euler: 1; GLM: 0 and 3), -1 none
+	R *cells;             // the chunk, in pinned host memory
+	long first, count;    // its cells, numbered over the ghosted buffer
+	int *flags;           // take_cells: [0] a real past the planes is not 0, [1] an out-of-plane momentum is not 0
+};
+constexpr int CELLS_BLOCK = 256;
+
+// ghosted coordinates of cell c
+template <typename R>
+__device__ __forceinline__ void cell_coords(const CellBuffer<R> &b, long c, int *cc) {
+	const int gx = b.n[0] + 2 * NG;
+	const int gy = b.dim > 1 ? b.n[1] + 2 * NG : 1;
+	const long row = c / gx;
+	cc[0] = (int)(c - row * gx) - NG;
+	cc[2] = (int)(row / gy) - (b.dim > 2 ? NG : 0);
+	cc[1] = (int)(row % gy) - (b.dim > 1 ? NG : 0);
+}
+
+// planes -> cells, ghosts filled as after the reference's boundary() (axis by
+// axis, a later axis wins)
+template <typename R>
+__global__ void __launch_bounds__(CELLS_BLOCK) give_cells_kernel(const CellBuffer<R> b) {
+	__shared__ __align__(16) R sh[CELLS_BLOCK * HYDRO_MAX_STATES];
+	const long base = (long)blockIdx.x * CELLS_BLOCK;
+	const int here = (int)min((long)CELLS_BLOCK, b.count - base);
+	const int t = threadIdx.x;
+	if (t < here) {
+		int cc[3];
+		cell_coords(b, b.first + base + t, cc);
+		Mapped m[3];
+#pragma unroll
+		for (int a = 0; a < 3; ++a) {
+			if (a < b.dim) m[a] = map_coord(cc[a], b.n[a], b.bc[2 * a], b.bc[2 * a + 1], 2 * a);
+			else { m[a].idx = 0; m[a].mirror = 0; m[a].fixedFace = -1; }
+		}
+		const long src = (long)m[0].idx + (long)b.n[0] * (m[1].idx + (long)b.n[1] * m[2].idx);
+		for (int f = 0; f < b.S; ++f) {
+			R v = f < b.q ? b.U[f * b.ps + src] : f < b.q + b.nstat ? b.stat[(f - b.q) * b.ps + src] : R(0);
+#pragma unroll
+			for (int a = 0; a < 3; ++a) {
+				if (m[a].fixedFace >= 0) v = b.fixedv[m[a].fixedFace][f];
+				else if (m[a].mirror && (f == b.vec1 + a || (b.vec2 >= 0 && f == b.vec2 + a))) v = -v;
+			}
+			sh[t * b.S + f] = v;
+		}
+	}
+	__syncthreads();
+	const int reals = here * b.S;
+	constexpr int PER = 16 / sizeof(R);
+	R *out = b.cells + base * b.S;     // 16-byte aligned: CELLS_BLOCK cells are a multiple of 16 bytes
+	for (int i = t * PER; i < reals; i += CELLS_BLOCK * PER) {
+		if (i + PER <= reals) {
+			*(int4 *)(out + i) = *(const int4 *)(sh + i);
+		} else {
+			for (int k = i; k < reals; ++k) out[k] = sh[k];
+		}
+	}
+}
+
+// cells -> planes, interior cells only
+template <typename R>
+__global__ void __launch_bounds__(CELLS_BLOCK) take_cells_kernel(const CellBuffer<R> b) {
+	__shared__ __align__(16) R sh[CELLS_BLOCK * HYDRO_MAX_STATES];
+	const long base = (long)blockIdx.x * CELLS_BLOCK;
+	const int here = (int)min((long)CELLS_BLOCK, b.count - base);
+	const int t = threadIdx.x;
+	const int reals = here * b.S;
+	constexpr int PER = 16 / sizeof(R);
+	const R *in = b.cells + base * b.S;
+	for (int i = t * PER; i < reals; i += CELLS_BLOCK * PER) {
+		if (i + PER <= reals) {
+			*(int4 *)(sh + i) = *(const int4 *)(in + i);
+		} else {
+			for (int k = i; k < reals; ++k) sh[k] = in[k];
+		}
+	}
+	__syncthreads();
+	bool past = false, outOfPlane = false;
+	if (t < here) {
+		int cc[3];
+		cell_coords(b, b.first + base + t, cc);
+		bool inside = true;
+#pragma unroll
+		for (int a = 0; a < 3; ++a)
+			if (a < b.dim) inside = inside && cc[a] >= 0 && cc[a] < b.n[a];
+		if (inside) {
+			const long dst = (long)cc[0] + (long)b.n[0] * (cc[1] + (long)b.n[1] * cc[2]);
+			for (int f = 0; f < b.S; ++f) {
+				const R v = sh[t * b.S + f];
+				if (f < b.q) b.U[f * b.ps + dst] = v;
+				else if (f < b.q + b.nstat) b.stat[(f - b.q) * b.ps + dst] = v;
+				else past = past || v != R(0);
+				if (f >= 1 + b.dim && f <= 3) outOfPlane = outOfPlane || v != R(0);
+			}
+		}
+	}
+	// every wave that found one writes the same 1
+	if (wave_any(past) && (t & 63) == 0) b.flags[0] = 1;
+	if (wave_any(outOfPlane) && (t & 63) == 0) b.flags[1] = 1;
+}
+
 // calcDT (eqn.lua:1187-1224 + calcDT.cl:38-73) and reduceMin: per-cell dt in
 // double, wave min, one atomic min per wave into dev->dtmin[slot].
 template <typename R, template <typename> class EQ, int DIM>

@@ -689,41 +689,6 @@ static void unpack_with_ghosts(const Grid &g, const R *planes, const R *stat, R 
 }
 
 template <typename R>
-static int grid_upload_t(Grid &g, const void *U, hipStream_t s) {
-	std::vector<R> planes((size_t)g.Q * g.ps), stat((size_t)g.NSTAT * g.ps);
-	pack_interior<R>(g, (const R *)U, planes.data(), stat.data());
-	HIPCHECK(hipMemcpyAsync(g.U[0], planes.data(), planes.size() * sizeof(R), hipMemcpyHostToDevice, s));
-	if (g.NSTAT) HIPCHECK(hipMemcpyAsync(g.stat, stat.data(), stat.size() * sizeof(R), hipMemcpyHostToDevice, s));
-	HIPCHECK(hipStreamSynchronize(s));
-	g.dtValid = 0;
-	return 0;
-}
-
-template <typename R>
-static int grid_download_t(const Grid &g, void *U, hipStream_t s) {
-	std::vector<R> planes((size_t)g.Q * g.ps), stat((size_t)g.NSTAT * g.ps);
-	HIPCHECK(hipMemcpyAsync(planes.data(), g.U[0], planes.size() * sizeof(R), hipMemcpyDeviceToHost, s));
-	if (g.NSTAT) HIPCHECK(hipMemcpyAsync(stat.data(), g.stat, stat.size() * sizeof(R), hipMemcpyDeviceToHost, s));
-	HIPCHECK(hipStreamSynchronize(s));
-	unpack_with_ghosts<R>(g, planes.data(), stat.data(), (R *)U);
-	return 0;
-}
-
-[[maybe_unused]] static int grid_upload(Grid &g, const void *U, size_t bytes, hipStream_t s) {
-	if (!U) return fail("NULL argument");
-	size_t need = ghosted_cells(g) * g.S * g.elem;
-	if (bytes != need) return fail("upload size %zu != %zu (numCells * numStates * sizeof(real))", bytes, need);
-	return g.elem == 8 ? grid_upload_t<double>(g, U, s) : grid_upload_t<float>(g, U, s);
-}
-
-[[maybe_unused]] static int grid_download(const Grid &g, void *U, size_t bytes, hipStream_t s) {
-	if (!U) return fail("NULL argument");
-	size_t need = ghosted_cells(g) * g.S * g.elem;
-	if (bytes != need) return fail("download size %zu != %zu (numCells * numStates * sizeof(real))", bytes, need);
-	return g.elem == 8 ? grid_download_t<double>(g, U, s) : grid_download_t<float>(g, U, s);
-}
-
-template <typename R>
 static GridArgs<R> grid_args(const Grid &g, int slot) {
 	GridArgs<R> a;
 	std::memset(&a, 0, sizeof a);

@@ -69,6 +69,13 @@ template <typename R>
 hipError_t launch_stats(int eqn, int dim, const GridDesc<R> &g, int field, KSum *partial, int nPartial, double nInterior,
 	double *out, const double *eqnPar /* gamma, rhoMin, PMin */, hipStream_t s);
 
+// one chunk of the ghosted cons_t buffer from (give) or to (take) the planes
+template <typename R> struct CellBuffer;
+template <typename R>
+hipError_t launch_give_cells(const CellBuffer<R> &b, hipStream_t s);
+template <typename R>
+hipError_t launch_take_cells(const CellBuffer<R> &b, hipStream_t s);
+
 hipError_t launch_reset_slots(DevScalars *dev, int mask, hipStream_t s);
 hipError_t launch_fold_slot(DevScalars *dev, int slot, hipStream_t s);
 

@@ -1,0 +1,280 @@
+// fv_transfer.h — host <-> device transfers of the plain and batched solvers:
+// the reference's ghosted cons_t buffer (cells, caller's memory) against the
+// planes of the interior on the device.
+//
+// The buffer goes through pinned slots, chunk by chunk: a kernel converts between
+// cells and planes while it crosses the bus (give_cells_kernel,
+// take_cells_kernel, fv_aux.h), and the host only copies whole chunks between the
+// caller's memory and the slots, on up to 8 threads with two slots each, so that
+// the copy of one chunk overlaps the bus time of others. What bounds a large
+// transfer is the host's copy (first touches of the caller's pages included).
+// Before, the host packed and unpacked the cells itself beside pageable copies of
+// all planes: down 256^2 FP64 .47 -> .19, 1024^2 13 -> 1.6, 256^3 FP32 107 -> 9.8;
+// up 1024^2 FP64 10.4 -> 1.3, 256^3 FP32 84 -> 10.6 ms (42 GB/s of the buffer).
+#pragma once
+
+#include <atomic>
+#include <condition_variable>
+#include <mutex>
+
+#include "fv_host.h"
+
+namespace hydro {
+
+// Pinned slots shared by every solver and batch of the process: at most
+// MAX_SLOTS, made as they are needed and freed with the last handle.
+class PinnedSlots {
+public:
+	static constexpr size_t SLOT = (size_t)2 << 20;
+	static constexpr int MAX_SLOTS = 16;
+
+	void add_handle() {
+		std::lock_guard<std::mutex> lock(mu);
+		++handles;
+	}
+	void drop_handle() {
+		std::lock_guard<std::mutex> lock(mu);
+		if (--handles > 0) return;
+		for (char *p : idle) ignore(hipHostFree(p));
+		made -= (int)idle.size();
+		idle.clear();
+	}
+	// Between 1 and `want` slots (waiting for one while all are taken); 0 if
+	// there are none and none can be made.
+	int take(int want, char **out) {
+		std::unique_lock<std::mutex> lock(mu);
+		for (;;) {
+			int n = 0;
+			while (n < want && !idle.empty()) {
+				out[n++] = idle.back();
+				idle.pop_back();
+			}
+			while (n < want && made < MAX_SLOTS) {
+				void *p = nullptr;
+				if (hipHostMalloc(&p, SLOT, hipHostMallocPortable) != hipSuccess || !p) {
+					(void)hipGetLastError();
+					break;
+				}
+				++made;
+				out[n++] = (char *)p;
+			}
+			if (n > 0 || made == 0) return n;
+			freed.wait(lock);
+		}
+	}
+	void give(char **slots, int n) {
+		{
+			std::lock_guard<std::mutex> lock(mu);
+			for (int i = 0; i < n; ++i) idle.push_back(slots[i]);
+		}
+		freed.notify_all();
+	}
+
+private:
+	std::mutex mu;
+	std::condition_variable freed;
+	std::vector<char *> idle;
+	int made = 0, handles = 0;
+};
+
+inline PinnedSlots &pinned_slots() {
+	static PinnedSlots *p = new PinnedSlots();   // outlives every handle
+	return *p;
+}
+
+// Below this the packed form (pageable copies of the planes) is as fast: 12 KB
+// take 25 us up and 35 down in it, 480 KB 98 and 170 against 43 and 59 through the
+// slots, most of them one launch and one event.
+static constexpr size_t CHUNKED_MIN = (size_t)96 << 10;
+
+template <typename R>
+static int upload_packed(Grid &g, const void *U, hipStream_t s) {
+	std::vector<R> planes((size_t)g.Q * g.ps), stat((size_t)g.NSTAT * g.ps);
+	pack_interior<R>(g, (const R *)U, planes.data(), stat.data());
+	HIPCHECK(hipMemcpyAsync(g.U[0], planes.data(), planes.size() * sizeof(R), hipMemcpyHostToDevice, s));
+	if (g.NSTAT) HIPCHECK(hipMemcpyAsync(g.stat, stat.data(), stat.size() * sizeof(R), hipMemcpyHostToDevice, s));
+	HIPCHECK(hipStreamSynchronize(s));
+	g.dtValid = 0;
+	return 0;
+}
+
+template <typename R>
+static int download_packed(const Grid &g, void *U, hipStream_t s) {
+	std::vector<R> planes((size_t)g.Q * g.ps), stat((size_t)g.NSTAT * g.ps);
+	HIPCHECK(hipMemcpyAsync(planes.data(), g.U[0], planes.size() * sizeof(R), hipMemcpyDeviceToHost, s));
+	if (g.NSTAT) HIPCHECK(hipMemcpyAsync(stat.data(), g.stat, stat.size() * sizeof(R), hipMemcpyDeviceToHost, s));
+	HIPCHECK(hipStreamSynchronize(s));
+	unpack_with_ghosts<R>(g, planes.data(), stat.data(), (R *)U);
+	return 0;
+}
+
+
+// g.ePot from the interior cells of an uploaded buffer
+template <typename R>
+static void keep_ePot(Grid &g, const R *aos) {
+	const int dim = g.dim, nx = g.n[0];
+	const long gx = nx + 2 * NG, gy = dim > 1 ? g.n[1] + 2 * NG : 1;
+	g.ePot.assign(g.ncell, 0.);
+	double *ePot = g.ePot.data();
+	parallel_ranges((long)g.n[1] * g.n[2], 64, [&](long r0, long r1) {
+		for (long row = r0; row < r1; ++row) {
+			const long j = row % g.n[1] + (dim > 1 ? NG : 0), k = row / g.n[1] + (dim > 2 ? NG : 0);
+			const R *u = aos + (size_t)(NG + gx * (j + gy * k)) * g.S;
+			for (int i = 0; i < nx; ++i) ePot[(size_t)nx * row + i] = (double)u[(size_t)i * g.S + 5];
+		}
+	});
+}
+
+template <typename R>
+static CellBuffer<R> cell_buffer(const Grid &g) {
+	CellBuffer<R> b;
+	std::memset(&b, 0, sizeof b);
+	b.U = (R *)g.U[0];
+	b.stat = (R *)g.stat;
+	b.ps = g.ps;
+	b.dim = g.dim;
+	b.q = g.Q;
+	b.nstat = g.NSTAT;
+	b.S = g.S;
+	for (int i = 0; i < 3; ++i) b.n[i] = g.n[i];
+	for (int f = 0; f < 6; ++f) {
+		b.bc[f] = g.cfg.boundary[f];
+		for (int j = 0; j < g.S; ++j) b.fixedv[f][j] = R(g.cfg.boundary_fixed[f][j]);
+	}
+	const bool glm = g.cfg.eqn == HYDRO_EQN_GLM_MAXWELL;
+	b.vec1 = glm ? 0 : 1;
+	b.vec2 = glm ? 3 : -1;
+	return b;
+}
+
+// Moves the ghosted buffer U (host) up to or down from g's planes through the
+// slots. flags (up): what take_cells found. Returns 1 if no slot could be had
+// (nothing was moved).
+template <typename R, bool UP>
+static int move_cells(const Grid &g, R *U, hipStream_t s, int *flags) {
+	const size_t cellBytes = (size_t)g.S * sizeof(R);
+	const long total = (long)ghosted_cells(g);
+	const size_t bytes = (size_t)total * cellBytes;
+	constexpr size_t FLAG_BYTES = 64;
+	const long maxCells = (long)((PinnedSlots::SLOT - FLAG_BYTES) / cellBytes) / CELLS_BLOCK * CELLS_BLOCK;
+	const long hw = std::max(1L, (long)std::thread::hardware_concurrency());
+	const long threads = std::max(1L, std::min({8L, hw, (long)(bytes >> 20)}));
+	// two chunks a thread at least, a slot's worth at most
+	long cells = (total + 2 * threads - 1) / (2 * threads);
+	cells = std::min(maxCells, (cells + CELLS_BLOCK - 1) / CELLS_BLOCK * CELLS_BLOCK);
+	const long chunks = (total + cells - 1) / cells;
+	char *slots[PinnedSlots::MAX_SLOTS];
+	const int nSlots = pinned_slots().take((int)std::min(2 * threads, chunks), slots);
+	if (nSlots < 1) return 1;
+	const long workers = std::max(1, nSlots / 2);
+	int device = 0;
+	hipError_t first = hipGetDevice(&device);
+	std::atomic<long> next{0};
+	std::atomic<int> err{(int)first};
+	int *const flagWords = (int *)(slots[0] + PinnedSlots::SLOT - FLAG_BYTES);
+	flagWords[0] = flagWords[1] = 0;
+	const CellBuffer<R> shape = cell_buffer<R>(g);
+	auto work = [&](long w, bool ownThread) {
+		auto ok = [&](hipError_t e) {
+			int none = hipSuccess;
+			if (e != hipSuccess) err.compare_exchange_strong(none, (int)e);
+			return e == hipSuccess;
+		};
+		if (ownThread && !ok(hipSetDevice(device))) return;
+		const int nb = std::min(2, nSlots - (int)(2 * w));
+		hipEvent_t ev[2] = {nullptr, nullptr};
+		long at[2] = {-1, -1};      // the chunk each slot holds (down) or last sent (up)
+		for (int i = 0; i < nb; ++i)
+			if (!ok(hipEventCreateWithFlags(&ev[i], hipEventDisableTiming))) ev[i] = nullptr;
+		auto drain = [&](int i) {   // the slot's kernel has ended; down: its cells go to the caller
+			if (at[i] < 0) return;
+			if (ok(hipEventSynchronize(ev[i])) && !UP) {
+				const long c0 = at[i] * cells, n = std::min(cells, total - c0);
+				std::memcpy((char *)U + (size_t)c0 * cellBytes, slots[2 * w + i], (size_t)n * cellBytes);
+			}
+			at[i] = -1;
+		};
+		int i = 0;
+		while (err.load() == hipSuccess) {
+			const long c = next.fetch_add(1);
+			if (c >= chunks) break;
+			drain(i);
+			CellBuffer<R> b = shape;
+			b.first = c * cells;
+			b.count = std::min(cells, total - b.first);
+			b.cells = (R *)slots[2 * w + i];
+			b.flags = flagWords;
+			if (UP) std::memcpy(b.cells, (const char *)U + (size_t)b.first * cellBytes, (size_t)b.count * cellBytes);
+			if (!ok(UP ? launch_take_cells<R>(b, s) : launch_give_cells<R>(b, s))) break;
+			if (!ok(hipEventRecord(ev[i], s))) {
+				ok(hipStreamSynchronize(s));     // the slot is still read or written
+				break;
+			}
+			at[i] = c;
+			i = i + 1 < nb ? i + 1 : 0;
+		}
+		drain(i);
+		drain(nb - 1 - i);
+		for (int k = 0; k < nb; ++k)
+			if (ev[k]) ignore(hipEventDestroy(ev[k]));
+	};
+	std::vector<std::thread> th;
+	th.reserve((size_t)workers);
+	for (long w = 1; w < workers; ++w) {
+		try {
+			th.emplace_back(work, w, true);
+		} catch (const std::system_error &) {
+			break;      // the chunks go to the threads there are
+		}
+	}
+	work(0, false);
+	for (auto &t : th) t.join();
+	if (flags) {
+		flags[0] = flagWords[0];
+		flags[1] = flagWords[1];
+	}
+	pinned_slots().give(slots, nSlots);
+	if (err.load() != hipSuccess) return fail("transfer of the cons_t buffer: %s", hipGetErrorString((hipError_t)err.load()));
+	return 0;
+}
+
+template <typename R>
+static int grid_upload_t(Grid &g, const void *U, size_t bytes, hipStream_t s) {
+	if (bytes < CHUNKED_MIN) return upload_packed<R>(g, U, s);
+	int flags[2] = {0, 0};
+	const int rc = move_cells<R, true>(g, (R *)const_cast<void *>(U), s, flags);
+	if (rc > 0) return upload_packed<R>(g, U, s);
+	if (rc < 0) return rc;
+	const bool euler = g.cfg.eqn == HYDRO_EQN_EULER;
+	// as pack_interior: out-of-plane momenta that are zero everywhere stay so;
+	// ePot is kept on the host where any is not 0
+	g.nvel = euler && g.dim < 3 && !flags[1] ? g.dim : 3;
+	g.ePot.clear();
+	if (euler && flags[0]) keep_ePot<R>(g, (const R *)U);
+	g.dtValid = 0;
+	return 0;
+}
+
+template <typename R>
+static int grid_download_t(const Grid &g, void *U, size_t bytes, hipStream_t s) {
+	// a state with ePot takes it from the host
+	if (bytes < CHUNKED_MIN || !g.ePot.empty()) return download_packed<R>(g, U, s);
+	const int rc = move_cells<R, false>(g, (R *)U, s, nullptr);
+	return rc > 0 ? download_packed<R>(g, U, s) : rc;
+}
+
+static int grid_upload(Grid &g, const void *U, size_t bytes, hipStream_t s) {
+	if (!U) return fail("NULL argument");
+	size_t need = ghosted_cells(g) * g.S * g.elem;
+	if (bytes != need) return fail("upload size %zu != %zu (numCells * numStates * sizeof(real))", bytes, need);
+	return g.elem == 8 ? grid_upload_t<double>(g, U, bytes, s) : grid_upload_t<float>(g, U, bytes, s);
+}
+
+static int grid_download(const Grid &g, void *U, size_t bytes, hipStream_t s) {
+	if (!U) return fail("NULL argument");
+	size_t need = ghosted_cells(g) * g.S * g.elem;
+	if (bytes != need) return fail("download size %zu != %zu (numCells * numStates * sizeof(real))", bytes, need);
+	return g.elem == 8 ? grid_download_t<double>(g, U, bytes, s) : grid_download_t<float>(g, U, bytes, s);
+}
+
+} // namespace hydro

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "fv_host.h"
+#include "fv_transfer.h"
 
 using namespace hydro;
 
@@ -74,12 +75,13 @@ extern "C" int hydro_create(const hydro_cfg *cfg, hydro_solver **out) {
 	int ndev = 0;
 	if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return fail("no HIP device available");
 	hydro_solver *h = new hydro_solver();
+	pinned_slots().add_handle();
 	grid_init(h->g, *cfg);
 	h->xcdRemap = 1;
 	auto cleanup = [&](int rc) { hydro_destroy(h); return rc; };
 	if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
-		delete h;
-		return fail("hipStreamCreate failed");
+		h->stream = nullptr;
+		return cleanup(fail("hipStreamCreate failed"));
 	}
 	size_t bytes = grid_bytes(h->g);
 	if (hipMalloc(&h->mem, bytes) != hipSuccess) return cleanup(fail("hipMalloc %zu B of solver state", bytes));
@@ -102,6 +104,7 @@ extern "C" int hydro_destroy(hydro_solver *h) {
 	if (h->totalsDev) ignore(hipFree(h->totalsDev));
 	if (h->stream) ignore(hipStreamDestroy(h->stream));
 	delete h;
+	pinned_slots().drop_handle();
 	return 0;
 }
 
@@ -451,6 +454,7 @@ extern "C" int hydro_batch_create(const hydro_cfg *cfgs, int n, hydro_batch **ou
 	int ndev = 0;
 	if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return fail("no HIP device available");
 	hydro_batch *b = new hydro_batch();
+	pinned_slots().add_handle();
 	b->grids.resize(n);
 	b->xcdRemap = 1;
 	b->wavesPerBlock = 4;
@@ -463,8 +467,8 @@ extern "C" int hydro_batch_create(const hydro_cfg *cfgs, int n, hydro_batch **ou
 	b->active.assign(n, 1);
 	auto cleanup = [&](int rc) { hydro_batch_destroy(b); return rc; };
 	if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) {
-		delete b;
-		return fail("hipStreamCreate failed");
+		b->stream = nullptr;
+		return cleanup(fail("hipStreamCreate failed"));
 	}
 	size_t total = 0;
 	for (auto &g : b->grids) {
@@ -494,6 +498,7 @@ extern "C" int hydro_batch_destroy(hydro_batch *b) {
 	if (b->descs) ignore(hipFree(b->descs));
 	if (b->stream) ignore(hipStreamDestroy(b->stream));
 	delete b;
+	pinned_slots().drop_handle();
 	return 0;
 }
 
