@@ -125,6 +125,31 @@ static void keep_ePot(Grid &g, const R *aos) {
 	});
 }
 
+// g.ePot into every cell of a downloaded buffer, ghosts as the other fields'
+template <typename R>
+static void put_ePot(const Grid &g, R *aos) {
+	int gs[3];
+	for (int i = 0; i < 3; ++i) gs[i] = i < g.dim ? g.n[i] + 2 * NG : 1;
+	const hydro_cfg &c = g.cfg;
+	parallel_ranges((long)gs[1] * gs[2], 64, [&](long r0, long r1) {
+		for (long row = r0; row < r1; ++row) {
+			const int at[3] = {0, (int)(row % gs[1]), (int)(row / gs[1])};
+			HostMap m[3] = {{0, 0, -1}, {0, 0, -1}, {0, 0, -1}};
+			for (int a = 1; a < g.dim; ++a)
+				m[a] = host_map(at[a] - NG, g.n[a], c.boundary[2 * a], c.boundary[2 * a + 1], 2 * a);
+			const double *src = g.ePot.data() + (size_t)g.n[0] * (m[1].idx + (size_t)g.n[1] * m[2].idx);
+			R *u = aos + (size_t)row * gs[0] * g.S + 5;
+			for (int i = 0; i < gs[0]; ++i, u += g.S) {
+				m[0] = host_map(i - NG, g.n[0], c.boundary[0], c.boundary[1], 0);
+				R v = R(src[m[0].idx]);
+				for (int a = 0; a < g.dim; ++a)
+					if (m[a].fixedFace >= 0) v = R(c.boundary_fixed[m[a].fixedFace][5]);
+				*u = v;
+			}
+		}
+	});
+}
+
 template <typename R>
 static CellBuffer<R> cell_buffer(const Grid &g) {
 	CellBuffer<R> b;
@@ -257,10 +282,11 @@ static int grid_upload_t(Grid &g, const void *U, size_t bytes, hipStream_t s) {
 
 template <typename R>
 static int grid_download_t(const Grid &g, void *U, size_t bytes, hipStream_t s) {
-	// a state with ePot takes it from the host
-	if (bytes < CHUNKED_MIN || !g.ePot.empty()) return download_packed<R>(g, U, s);
+	if (bytes < CHUNKED_MIN) return download_packed<R>(g, U, s);
 	const int rc = move_cells<R, false>(g, (R *)U, s, nullptr);
-	return rc > 0 ? download_packed<R>(g, U, s) : rc;
+	if (rc > 0) return download_packed<R>(g, U, s);
+	if (rc == 0 && !g.ePot.empty()) put_ePot<R>(g, (R *)U);
+	return rc;
 }
 
 static int grid_upload(Grid &g, const void *U, size_t bytes, hipStream_t s) {
