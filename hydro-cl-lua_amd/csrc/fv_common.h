@@ -60,7 +60,8 @@ struct DevScalars {
 	double t;
 	double dt;
 	unsigned nonFinite;       // set by nonfinite_kernel
-	unsigned pad0[3];
+	unsigned pad0[2];
+	unsigned ticket;          // blocks of a statistics pass that have finished, 0 between launches
 	double pad[4];
 };
 

@@ -63,11 +63,12 @@ hipError_t launch_nonfinite(const R *U, const R *stat, long ps, long ncell, int 
 template <typename R>
 hipError_t launch_totals(const R *U, long ps, long ncell, int q, KSum *partial, int nPartial, double *out, hipStream_t s);
 
-// min, max, average, standard deviation of one stored field (out: 4 doubles
-// on the device; partial: 2 nPartial KSums)
+// min, max, average, standard deviation of one field: 4 doubles to host (pinned
+// memory) where given, else to out (4 doubles on the device, used either way);
+// partial: 2 maxPartial KSums
 template <typename R>
-hipError_t launch_stats(int eqn, int dim, const GridDesc<R> &g, int field, KSum *partial, int nPartial, double nInterior,
-	double *out, const double *eqnPar /* gamma, rhoMin, PMin */, hipStream_t s);
+hipError_t launch_stats(int eqn, int dim, const GridDesc<R> &g, int field, KSum *partial, int maxPartial, double nInterior,
+	double *out, double *host, const double *eqnPar /* gamma, rhoMin, PMin */, hipStream_t s);
 
 // one chunk of the ghosted cons_t buffer from (give) or to (take) the planes
 template <typename R> struct CellBuffer;
