@@ -140,6 +140,8 @@ struct StageArgs {
 	int resetSlot;            // slot to clear to +inf, -1 none
 	int reduceSlot;           // slot to min-reduce the new state's dt into, -1 none
 	int advanceTime;          // t += dt, dt stored
+	double rkAlpha[4][4], rkBeta[4][4];   // the whole table, its order, and the steps of the launch (step1d_kernel)
+	int order, steps;
 	int tile;                 // plain 2D launch of the tile kernel (fv_tile.h)
 	int shareEdges;           // plain 2D launch: one strip-edge pass per block of 4 x-adjacent strips
 	int stepInTick;           // batch: skip grids with stepsLeft <= stepInTick

@@ -45,7 +45,7 @@ hipError_t launch_stage(const StageKey &k, const StageArgs<R> &a, dim3 grid, dim
 extern thread_local int stage_occupancy;
 // The same for one math policy, dimension and form (launch_stage picks by k.fast,
 // k.dim and the launch); each is defined in a translation unit of its own.
-enum { FORM_PLAIN = 0, FORM_TILE = 1, FORM_BATCH = 2 };
+enum { FORM_PLAIN = 0, FORM_TILE = 1, FORM_BATCH = 2, FORM_STEP = 3 };
 template <typename R, bool FAST, int DIM, int FORM>
 hipError_t launch_stage_dim(const StageKey &k, const StageArgs<R> &a, dim3 grid, dim3 block, hipStream_t s);
 

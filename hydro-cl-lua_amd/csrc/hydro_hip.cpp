@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "fv_host.h"
+#include "fv_step1d.h"
 #include "fv_transfer.h"
 
 using namespace hydro;
@@ -187,10 +188,61 @@ static int solver_stage(hydro_solver *h, int s, int useSlot, double hostDt, int 
 	return 0;
 }
 
+// 1D grids whose steps are one launch each (fv_step1d.h)
+static bool whole_steps(const Grid &g) {
+	return g.dim == 1 &&
+		(g.cfg.boundary[0] == HYDRO_BC_PERIODIC) == (g.cfg.boundary[1] == HYDRO_BC_PERIODIC);
+}
+// ... and of those, the ones that take several steps per launch, in one block
+static bool one_block(const Grid &g) { return g.n[0] <= step1d_out(g.rk.order) * STEP1D_WAVES; }
+static constexpr int STEPS_PER_LAUNCH = 256;     // keeps a launch under a millisecond or two
+
+// `steps` integrator steps of a 1D grid in one launch (more than one: one_block).
+template <typename R>
+static int solver_step1d(hydro_solver *h, int steps, int useSlot, double hostDt, int update, std::vector<hipEvent_t> *evs) {
+	Grid &g = h->g;
+	const int cur = g.slot, fixed = g.cfg.use_fixed_dt;
+	StageArgs<R> a;
+	stage_args<R>(g, 0, a);
+	grid_desc<R>(g, a.g);
+	a.steps = steps;
+	a.src = 0;
+	a.out = g.rk.order == 1 ? -1 : 1;      // the other buffer: neighbours read this one
+	if (useSlot) a.dtSlot = cur;
+	else a.hostDt = hostDt;
+	if (update && !fixed) {
+		a.reduceSlot = (cur + steps) % 3;
+		a.resetSlot = (cur + 2) % 3;       // (one block: it leaves all three slots as they belong)
+	}
+	a.advanceTime = update;
+	a.xcdRemap = h->xcdRemap;
+	const long waves = (g.n[0] + step1d_out(g.rk.order) - 1) / step1d_out(g.rk.order);
+	const int perBlock = steps > 1 ? (int)waves : 4;
+	a.nBlocks = (int)((waves + perBlock - 1) / perBlock);
+	hipEvent_t e0 = nullptr, e1 = nullptr;
+	if (evs) {
+		HIPCHECK(hipEventCreate(&e0));
+		HIPCHECK(hipEventCreate(&e1));
+		evs->push_back(e0);
+		evs->push_back(e1);
+		HIPCHECK(hipEventRecord(e0, h->stream));
+	}
+	hipError_t e = launch_stage<R>(stage_key(g), a, dim3(a.nBlocks), dim3(WAVE * perBlock), h->stream);
+	if (e != hipSuccess) return fail("step kernel launch: %s", hipGetErrorString(e));
+	if (evs) HIPCHECK(hipEventRecord(e1, h->stream));
+	if (steps == 1) std::swap(g.U[0], g.rk.order == 1 ? g.ping : g.U[1]);
+	if (update && !fixed) {
+		g.slot = (cur + steps) % 3;
+		g.dtValid = 1;
+	}
+	return 0;
+}
+
 // One integrator step. useSlot: dt = cfl * dtmin[slot] on the device.
 template <typename R>
 static int solver_step(hydro_solver *h, int useSlot, double hostDt, int update, std::vector<hipEvent_t> *evs) {
 	Grid &g = h->g;
+	if (whole_steps(g)) return solver_step1d<R>(h, 1, useSlot, hostDt, update, evs);
 	int o = g.rk.order;
 	int cur = g.slot;
 	int fixed = g.cfg.use_fixed_dt;
@@ -231,7 +283,16 @@ static int update_impl(hydro_solver *h, int nsteps, std::vector<hipEvent_t> *evs
 		if (grid_dt_kernel(g, g.slot, h->stream)) return -1;
 		g.dtValid = 1;
 	}
-	for (int i = 0; i < nsteps; ++i) {
+	const bool several = whole_steps(g) && one_block(g) && !evs;
+	for (int i = 0; i < nsteps;) {
+		const int steps = several ? std::min(nsteps - i, STEPS_PER_LAUNCH) : 1;
+		i += steps;
+		if (steps > 1) {
+			const int rc = g.elem == 8 ? solver_step1d<double>(h, steps, !fixed, g.cfg.fixed_dt, 1, nullptr)
+			                           : solver_step1d<float>(h, steps, !fixed, g.cfg.fixed_dt, 1, nullptr);
+			if (rc) return rc;
+			continue;
+		}
 		int rc = g.elem == 8 ? solver_step<double>(h, !fixed, g.cfg.fixed_dt, 1, evs)
 		                     : solver_step<float>(h, !fixed, g.cfg.fixed_dt, 1, evs);
 		if (rc) return rc;
