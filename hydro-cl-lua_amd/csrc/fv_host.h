@@ -231,76 +231,110 @@ static long device_cus() {
 
 static StageKey stage_key_cfg(const hydro_cfg &cfg, int nvel);
 
-// Blocks of the plain FP64 stage kernel of cfg that a CU holds at once (its
-// registers and LDS decide: the heavier reconstructions and fluxes hold 2 or
-// 3 where 'plm cons' with Roe holds 4); 4 if the query fails. The velocity
-// components are taken as the dimension's, the usual Euler state.
-static long plain_occupancy(const hydro_cfg &cfg) {
-	StageArgs<double> a{};
+// Blocks of the stage kernel of cfg that a CU holds at once (its registers and
+// LDS decide), from an occupancy query: 4 waves a block, or the batched kernel
+// with the given waves; 4 if the query fails. The velocity components are taken
+// as the dimension's, the usual Euler state.
+template <typename R>
+static long stage_blocks_per_cu(const hydro_cfg &cfg, int batchWaves) {
+	StageArgs<R> a{};
 	const StageKey k = stage_key_cfg(cfg, std::min(cfg.dim, 3));
 	stage_occupancy = 0;
-	if (launch_stage<double>(k, a, dim3(0), dim3(0), nullptr) != hipSuccess || stage_occupancy < 1) {
+	if (launch_stage<R>(k, a, dim3(0), dim3(WAVE * batchWaves), nullptr) != hipSuccess || stage_occupancy < 1) {
 		(void)hipGetLastError();
 		return 4;
 	}
 	return stage_occupancy;
 }
+static long stage_occupancy_of(const hydro_cfg &cfg, int batchWaves) {
+	return cfg.precision == HYDRO_REAL_F32 ? stage_blocks_per_cu<float>(cfg, batchWaves)
+	                                       : stage_blocks_per_cu<double>(cfg, batchWaves);
+}
 
-// Rows per wave of the plain stage kernel (2D), from KH sweeps (rows 3..32 at
-// 512^2 .. 4096^2, fast math). Each wave marches `rows` rows of a strip after a
-// warm-up of 1-3 rows and, in the 64-column strips, its strip-edge pass (about
-// 1.5 rows of work; about 0.5 when a block's four x-adjacent strips share one
-// pass); halo strips (equations with a source) have no edge pass.
-// FP64: blocks of 4 waves are dealt to the CUs, a CU runs L = ceil(blocks /
-// CUs) of them, at most occ at once (the kernel's resident blocks per CU, from
-// an occupancy query), and the launch takes about
-// L * (rows + warm + edge) / eff(min(L, occ)), eff (fitted: .7, .77, .9, 1 for
-// 1, 2, 3, 4+) being how well that many waves per SIMD hide latency; the rows
-// in 4..8 with the least time are taken: for the kernels of 4 waves per SIMD 4
-// at 512^2 and 1024^2 (one round), 8 at 2048^2 and 4096^2. A halo-strip kernel
-// of at most 2 blocks per CU takes rows up to 16, so that its launch can end in
-// fewer rounds (GLM-Maxwell: 10 rows at 1024^2, 12 at 2048^2, each the fastest
-// of a sweep of 3..16). FP32 is latency-bound and gains from many short waves:
-// rows = clamp(strips * ny / 4096, 4, 8) (4 at 512^2 .. 1024^2, 8 from 2048^2;
-// longer waves leave a costly partial last round).
+// The marching kernel's time, but for a constant: L waves for each SIMD, of which
+// it holds occ at once, march `rows` (warm-up and edge pass included) each. k
+// waves together take 3 + k where one takes 4: a row is a chain of dependent
+// loads, square roots and divisions, and one wave alone fills a quarter of its
+// SIMD. (Measured, a row of FP32 'plm cons': 2.0, 2.65, 3.1, 3.4 us for 1..4
+// waves.)
+static double march_cost(long L, long occ, double rows) {
+	const long rem = L % occ;
+	return rows * ((double)(L / occ) * (3. + (double)occ) + (rem ? 3. + (double)rem : 0.));
+}
+
+// Rows a wave marches before or beside its own: the warm-up, and in the
+// 64-column strips the edge pass, about 1.5 rows of work (.5 where four waves of
+// a block share one).
+static double march_overhead(const hydro_cfg &cfg, bool shared) {
+	const int warm = cfg.plm ? 2 : (cfg.flux_limiter ? 3 : 1);
+	const bool edges = strip_edges(cfg.dim, eqn_has_source(cfg.eqn));
+	return warm + (!edges ? 0. : shared ? .5 : 1.5);
+}
+
+static long grid_strips(const hydro_cfg &cfg) {
+	const int so = strip_out(strip_edges(cfg.dim, eqn_has_source(cfg.eqn)));
+	return (cfg.size[0] + so - 1) / so;
+}
+
+// Rows per wave of the plain marching kernel: in 2D those in 2..8 of the least
+// march_cost. Short waves fill a grid that leaves SIMDs idle, long ones save
+// warm-ups, and the last round of waves should be a full one; beyond 8 nothing
+// is gained at 2048^2 and 4096^2, but a halo-strip kernel of at most 2 blocks
+// per CU takes up to 16, so that its launch can end in fewer rounds
+// (GLM-Maxwell FP64: 10 rows at 1024^2, 12 at 2048^2). us per stage at the rows
+// taken (against 4..8 by an older fit): shallow water 700x500 17.5 (19.3),
+// GLM-Maxwell FP32 512^2 14.3 (15.1), 700^2 17.4 (19.6), KH FP64 700^2 19.3 (23.5);
+// over 26 uneven shapes of all equations the rows taken were within 4 % of the
+// best of 2..16, most of them the best.
 // 3D: planes per block chunk (at most 16). Blocks are small (4 waves) and many resident
 // per CU, so the tail matters less than in 2D: keep at least 5000 blocks and,
 // among those chunk sizes, the fewest plane iterations per column (chunks that
 // divide the depth evenly, each with its 1-3 plane warm-up).
-static int default_rows(const hydro_cfg &cfg, int nx, int ny, int nz) {
+static int default_rows(const hydro_cfg &cfg) {
 	if (cfg.dim < 2) return 1;
-	const int so = strip_out(strip_edges(cfg.dim, eqn_has_source(cfg.eqn)));
-	long stripsX = (nx + so - 1) / so;
-	int warm = cfg.plm ? 2 : (cfg.flux_limiter ? 3 : 1);
+	const long stripsX = grid_strips(cfg), ny = cfg.size[1];
 	if (cfg.dim == 3) {
+		const int warm = cfg.plm ? 2 : (cfg.flux_limiter ? 3 : 1);
 		long W = cfg.precision == HYDRO_REAL_F32 ? Block3<float>::W : Block3<double>::W;
 		long perPlane = stripsX * ((ny + W - 1) / W);
 		long best = 8, bestCost = -1;
 		for (long r = 8; r <= EDGE_PLANES; ++r) {
-			long chunks = (nz + r - 1) / r;
+			long chunks = (cfg.size[2] + r - 1) / r;
 			if (r > 8 && perPlane * chunks < 5000) continue;
 			long cost = chunks * (r + warm);
 			if (bestCost < 0 || cost < bestCost) { best = r; bestCost = cost; }
 		}
 		return (int)best;
 	}
-	if (cfg.precision == HYDRO_REAL_F32)
-		return (int)std::max(4L, std::min(8L, (stripsX * (long)ny + 4095) / 4096));
-	static const double eff[5] = {0, .7, .77, .9, 1.};
-	const long cus = device_cus();
-	const long occ = plain_occupancy(cfg);
+	const long cus = device_cus(), occ = stage_occupancy_of(cfg, 0);
 	const bool edges = strip_edges(cfg.dim, eqn_has_source(cfg.eqn));
-	int best = 4;
-	double bestT = -1;
-	// at most 8 rows for 64-column strips and for kernels of 3 or more blocks
-	// per CU: longer strips measured no faster at 2048^2 and 4096^2
 	const int rMax = !edges && occ <= 2 ? 16 : 8;
-	for (int r = 4; r <= rMax; ++r) {
-		long blocks = (stripsX * ((ny + r - 1) / r) + 3) / 4;
-		long L = (blocks + cus - 1) / cus;
-		// the edge pass: a wave's own, or a quarter of its block's shared one
-		const double edge = !edges ? 0. : stripsX % 4 == 0 && 5 * r <= WAVE ? .5 : 1.5;
-		double t = (double)L * (r + warm + edge) / eff[std::min(std::min(L, occ), 4L)];
+	int best = 2;
+	double bestT = -1;
+	for (int r = 2; r <= rMax; ++r) {
+		const long blocks = (stripsX * ((ny + r - 1) / r) + 3) / 4;
+		const double t = march_cost((blocks + cus - 1) / cus, occ,
+			r + march_overhead(cfg, stripsX % 4 == 0 && 5 * r <= WAVE));
+		if (bestT < 0 || t < bestT * (1 - 1e-9)) { best = r; bestT = t; }
+	}
+	return best;
+}
+
+// Rows per wave of a batched launch over 2D grids of one configuration: by the
+// same cost, 2..32 rows. waves: of a block, perCU: such blocks resident on a CU.
+// Within 5 % of the best of 2..32 on ensembles of 4 to 64 grids, both precisions;
+// us per stage (at rows from the mean load): 48 FP32 grids of 64..512 78 (95), 24
+// 47 (61), 24 GLM-Maxwell FP32 33 (45), 24 FP64 62 (90).
+static int batch_rows(const std::vector<const hydro_cfg *> &grids, int waves, long perCU) {
+	const hydro_cfg &cfg = *grids[0];
+	if (cfg.dim < 2) return 1;
+	const long simds = 4 * (long)device_cus(), occ = std::max(1L, perCU * waves / 4);
+	int best = 2;
+	double bestT = -1;
+	for (int r = 2; r <= EDGE_ROWS; ++r) {
+		long items = 0;
+		for (const hydro_cfg *c : grids) items += grid_strips(*c) * ((c->size[1] + r - 1) / r);
+		const double t = march_cost((items + simds - 1) / simds, occ, r + march_overhead(cfg, false));
 		if (bestT < 0 || t < bestT * (1 - 1e-9)) { best = r; bestT = t; }
 	}
 	return best;
@@ -318,17 +352,19 @@ static long tile_blocks(const hydro_cfg &cfg) {
 
 // Whether the plain 2D solver takes the tile kernel (fv_tile.h) and not the
 // marching one. Its time is about 5.2 us plus 1.4-1.8 us (IEEE 3) for each block
-// a CU has to run; the marching kernel's is flat (FAST 10-27 us, IEEE 22-35 us, by
-// the scheme) while its waves are all resident at once and then grows at half to
-// two thirds of that rate. Measured at 4 blocks per CU (384^2), tile / marching:
-// 'plm cons' FP64 10.4 / 13.8, FP32 8.9 / 11.5, flux-limited 11.6 / 15.7, shallow
-// water 11.4 / 13.9, GLM-Maxwell FP32 10.2 / 12.2, FP64 14.2 / 14.3, HLLC 11.7 /
-// 17.1, 'plm athena' 18.3 / 27.1 us; 'plm cons' at 5.3 (512^2) 15.0 / 14.8. IEEE at
+// a CU has to run; the marching kernel's is flat (FAST 9-14 us at 2 or 3 rows, IEEE
+// 22-35 us, by the scheme) while its waves are all resident at once and then grows at
+// half to two thirds of that rate. Measured at 4 blocks per CU (384^2), tile /
+// marching at its best rows: 'plm cons' FP64 10.6 / 12.5, FP32 9.3 / 10.6, van Leer
+// 10.1 / 12.0, flux-limited 11.7 / 14.0, shallow water 11.5 / 12.1, GLM-Maxwell FP32
+// 10.6 / 10.7; at 256^2 7.8 / 10.6, 7.2 / 9.7, 7.8 / 10.7, 8.6 / 12.0, 8.1 / 9.5,
+// 7.4 / 8.8; 'plm cons' at 5.3 (512^2) 15.0 / 14.8. GLM-Maxwell FP64, twelve state
+// components in 64 bits, 8.9 / 9.9 at 1.7 (256^2), 10.8 / 10.5 at 2.5 (320^2). IEEE at
 // 14 (about 830^2): 47.1 / 50.9 at 800^2.
 static bool tile_form(const hydro_cfg &cfg) {
 	if (cfg.dim != 2) return false;
 	const bool heavy = cfg.eqn == HYDRO_EQN_GLM_MAXWELL && cfg.precision == HYDRO_REAL_F64;
-	const double perCU = !cfg.fast_math ? 14. : heavy ? 4. : 4.5;
+	const double perCU = !cfg.fast_math ? 14. : heavy ? 2.4 : 4.5;
 	return (double)tile_blocks(cfg) <= perCU * (double)device_cus();
 }
 
@@ -353,8 +389,8 @@ static void grid_init(Grid &g, const hydro_cfg &cfg) {
 	g.slot = 0;
 	g.dtValid = 0;
 	g.nvel = 3;
-	g.rowsPerWave = default_rows(cfg, g.n[0], g.n[1], g.n[2]);
-	g.tile = tile_form(cfg);
+	g.rowsPerWave = 1;       // the caller's to set, as the form is
+	g.tile = 0;
 }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }

@@ -38,8 +38,9 @@ inline int limiter_template_id(int index) {
 template <typename R> struct GridArgs;
 
 // grid.x > 0: plain launch of that many blocks; grid.x == 0: persistent
-// batched launch over a.grids; grid.x == 0 and block.x == 0: no launch, the
-// plain kernel's resident blocks per CU go to stage_occupancy (this thread's).
+// batched launch over a.grids; grid.x == 0 and block.x == 0, or no items: no
+// launch, the plain or batched kernel's resident blocks per CU go to
+// stage_occupancy (this thread's).
 template <typename R>
 hipError_t launch_stage(const StageKey &k, const StageArgs<R> &a, dim3 grid, dim3 block, hipStream_t s);
 extern thread_local int stage_occupancy;

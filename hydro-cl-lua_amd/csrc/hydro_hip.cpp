@@ -78,6 +78,8 @@ extern "C" int hydro_create(const hydro_cfg *cfg, hydro_solver **out) {
 	hydro_solver *h = new hydro_solver();
 	pinned_slots().add_handle();
 	grid_init(h->g, *cfg);
+	h->g.rowsPerWave = default_rows(*cfg);
+	h->g.tile = tile_form(*cfg);
 	h->xcdRemap = 1;
 	auto cleanup = [&](int rc) { hydro_destroy(h); return rc; };
 	if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
@@ -511,6 +513,15 @@ static int batch_step(hydro_batch *b, int cur) {
 	return 0;
 }
 
+// rows per wave by the batch's load
+static int batch_rows_of(const hydro_batch *b) {
+	const hydro_cfg &cfg = b->grids[0].cfg;
+	if (cfg.dim < 2) return 1;
+	std::vector<const hydro_cfg *> shapes;
+	for (auto &g : b->grids) shapes.push_back(&g.cfg);
+	return batch_rows(shapes, b->wavesPerBlock, stage_occupancy_of(cfg, b->wavesPerBlock));
+}
+
 extern "C" int hydro_batch_create(const hydro_cfg *cfgs, int n, hydro_batch **out) {
 	if (!out) return fail("out is NULL");
 	*out = nullptr;
@@ -529,12 +540,8 @@ extern "C" int hydro_batch_create(const hydro_cfg *cfgs, int n, hydro_batch **ou
 	b->grids.resize(n);
 	b->xcdRemap = 1;
 	b->wavesPerBlock = 4;
-	long cells = 0;
-	for (int i = 0; i < n; ++i) {
-		grid_init(b->grids[i], cfgs[i]);
-		cells += b->grids[i].ncell;
-	}
-	b->rowsPerWave = cfgs[0].dim >= 2 ? (int)std::max(4L, std::min(32L, cells / (64L * 4096) + 1)) : 1;
+	for (int i = 0; i < n; ++i) grid_init(b->grids[i], cfgs[i]);
+	b->rowsPerWave = batch_rows_of(b);
 	b->active.assign(n, 1);
 	auto cleanup = [&](int rc) { hydro_batch_destroy(b); return rc; };
 	if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) {
@@ -748,11 +755,12 @@ extern "C" int hydro_batch_time_updates(hydro_batch *b, int nsteps, int use_grap
 extern "C" int hydro_batch_autotune(hydro_batch *b, int trial_steps, int *rows_out, int *waves_out, double *ms_out) {
 	if (!b) return fail("NULL handle");
 	if (trial_steps < 1) trial_steps = 3;
-	static const int rowsCand[] = {2, 3, 4, 6, 8, 12, 16};
+	bool twoD = b->grids[0].dim >= 2;
+	// the rows by load first: 2 rows are worth trying only where they are those
+	const int rowsCand[] = {twoD ? batch_rows_of(b) : 2, 3, 4, 6, 8, 12, 16};
 	static const int wavesCand[] = {4, 2, 1};
 	int bestR = b->rowsPerWave, bestW = b->wavesPerBlock;
 	double best = 1e300;
-	bool twoD = b->grids[0].dim >= 2;
 	for (int w : wavesCand) {
 		for (int r : rowsCand) {
 			if (!twoD && r != rowsCand[0]) continue;
