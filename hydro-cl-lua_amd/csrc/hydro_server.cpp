@@ -12,9 +12,11 @@
 // on the device and the copy of the final state into pinned memory; an event
 // closes the chunk. No call waits for the whole device: a tick completes the
 // chunks whose events have fired (results unpacked, memory released), admits,
-// and starts the next chunk of every idle pool, so one pool's host work
-// overlaps the others' kernels; only when nothing can move does it wait, for
-// the chunk started first. A request's result does not depend on what else is
+// and starts the next chunk of every pool with fewer than two in flight: the
+// second is there when the first ends, whatever the host is doing then (a pool
+// sat idle for 1.3 ms of every 2.2 while the host launched for others and
+// unpacked results). Only when nothing can move does a tick wait, for the
+// chunk started first. A request's result does not depend on what else is
 // resident: per-grid dt and time, no arithmetic across grids.
 #include <deque>
 #include <map>
@@ -89,21 +91,25 @@ struct Request {
 	double t = 0;
 };
 
+struct Chunk {
+	std::vector<long long> landing;    // uploaded by the chunk (staging still held)
+	std::vector<long long> retiring;   // copied out by the chunk
+	void *descs = nullptr;             // device GridDesc array
+	size_t descCap = 0;
+	char *hostDescs = nullptr;         // pinned, written only while the chunk is not in flight
+	size_t hostDescCap = 0;
+	hipEvent_t done = nullptr;         // closes the chunk
+	bool inflight = false;
+	long long started = 0;             // launch order of the chunk in flight
+};
+
 struct Pool {
 	hydro_cfg cfg;
 	int nvel = 3;
 	std::vector<long long> joining;    // packed, uploaded by the pool's next chunk
 	std::vector<long long> resident;   // on the device, advanced by the next chunk
-	std::vector<long long> landing;    // uploaded by the chunk in flight (staging still held)
-	std::vector<long long> retiring;   // copied out by the chunk in flight
-	void *descs = nullptr;             // device GridDesc array
-	size_t descCap = 0;
-	char *hostDescs = nullptr;         // pinned, written only while the pool is idle
-	size_t hostDescCap = 0;
+	Chunk chunks[2];                   // in flight, one behind the other on the stream
 	hipStream_t stream = nullptr;
-	hipEvent_t done = nullptr;         // closes the chunk in flight
-	bool inflight = false;
-	long long started = 0;             // launch order of the chunk in flight
 	int slot = 0;
 	int rowsPerWave = 0;               // 0: by the load of each chunk
 	int wavesPerBlock = 1;
@@ -182,9 +188,11 @@ extern "C" int hydro_server_destroy(hydro_server *s) {
 			ignore(hipStreamSynchronize(p.stream));
 			ignore(hipStreamDestroy(p.stream));
 		}
-		if (p.done) ignore(hipEventDestroy(p.done));
-		if (p.descs) ignore(hipFree(p.descs));
-		if (p.hostDescs) ignore(hipHostFree(p.hostDescs));
+		for (auto &c : p.chunks) {
+			if (c.done) ignore(hipEventDestroy(c.done));
+			if (c.descs) ignore(hipFree(c.descs));
+			if (c.hostDescs) ignore(hipHostFree(c.hostDescs));
+		}
 	}
 	if (s->pinnedMem) ignore(hipHostFree(s->pinnedMem));
 	if (s->mem) ignore(hipFree(s->mem));
@@ -237,10 +245,12 @@ static int pool_for(hydro_server *s, const Request &r) {
 	p.rowsPerWave = r.g.dim >= 2 ? s->rowsPerWave : 1;
 	p.wavesPerBlock = s->wavesPerBlock;
 	if (hipStreamCreateWithFlags(&p.stream, hipStreamNonBlocking) != hipSuccess) return fail("hipStreamCreate failed");
-	if (hipEventCreateWithFlags(&p.done, hipEventDisableTiming) != hipSuccess) {
-		ignore(hipStreamDestroy(p.stream));
-		return fail("hipEventCreate failed");
-	}
+	for (auto &c : p.chunks)
+		if (hipEventCreateWithFlags(&c.done, hipEventDisableTiming) != hipSuccess) {
+			if (p.chunks[0].done) ignore(hipEventDestroy(p.chunks[0].done));
+			ignore(hipStreamDestroy(p.stream));
+			return fail("hipEventCreate failed");
+		}
 	s->pools.push_back(std::move(p));
 	return (int)s->pools.size() - 1;
 }
@@ -333,20 +343,21 @@ static int enqueue_retire(hydro_server *s, Pool &p, Request &r) {
 	return 0;
 }
 
-// One chunk of an idle pool on its stream: the joining requests' uploads, up
+// One chunk of a pool on its stream, behind the one in flight if there is one
+// (c is not): the joining requests' uploads, up
 // to steps_per_tick steps of every resident grid with steps left, the
 // copy-out of every request with none left (as far as staging allows: the
 // others wait for a later chunk), and the event that closes the chunk.
 // Returns 1 when it enqueued anything, 0 when there was nothing to do.
 template <typename R>
-static int launch_chunk(hydro_server *s, Pool &p) {
+static int launch_chunk(hydro_server *s, Pool &p, Chunk &c) {
 	bool any = false;
 	for (long long id : p.joining) {
 		Request &r = s->reqs.at(id);
 		if (enqueue_join(s, p, r)) return -1;
 		r.state = RESIDENT;
 		p.resident.push_back(id);
-		p.landing.push_back(id);
+		c.landing.push_back(id);
 		any = true;
 	}
 	p.joining.clear();
@@ -356,22 +367,22 @@ static int launch_chunk(hydro_server *s, Pool &p) {
 	const int n = (int)active.size();
 	if (n) {
 		const size_t descBytes = sizeof(GridDesc<R>) * n;
-		if (descBytes > p.descCap) {
-			// the pool is idle: nothing of its stream reads the old array
-			if (p.descs) HIPCHECK(hipFree(p.descs));
-			p.descs = nullptr;
-			p.descCap = 0;
+		if (descBytes > c.descCap) {
+			// nothing in flight reads this chunk's old array
+			if (c.descs) HIPCHECK(hipFree(c.descs));
+			c.descs = nullptr;
+			c.descCap = 0;
 			const size_t cap = std::max(descBytes * 2, (size_t)4096);
-			HIPCHECK(hipMalloc(&p.descs, cap));
-			p.descCap = cap;
+			HIPCHECK(hipMalloc(&c.descs, cap));
+			c.descCap = cap;
 		}
-		if (descBytes > p.hostDescCap) {
-			if (p.hostDescs) HIPCHECK(hipHostFree(p.hostDescs));
-			p.hostDescs = nullptr;
-			p.hostDescCap = 0;
+		if (descBytes > c.hostDescCap) {
+			if (c.hostDescs) HIPCHECK(hipHostFree(c.hostDescs));
+			c.hostDescs = nullptr;
+			c.hostDescCap = 0;
 			const size_t cap = std::max(descBytes * 2, (size_t)4096);
-			HIPCHECK(hipHostMalloc((void **)&p.hostDescs, cap, hipHostMallocDefault));
-			p.hostDescCap = cap;
+			HIPCHECK(hipHostMalloc((void **)&c.hostDescs, cap, hipHostMallocDefault));
+			c.hostDescCap = cap;
 		}
 		int rows = p.rowsPerWave;
 		if (!rows) {
@@ -382,7 +393,7 @@ static int launch_chunk(hydro_server *s, Pool &p) {
 			for (long long id : active) shapes.push_back(&s->reqs.at(id).cfg);
 			rows = batch_rows(shapes, p.wavesPerBlock, p.perCU);
 		}
-		GridDesc<R> *d = (GridDesc<R> *)p.hostDescs;
+		GridDesc<R> *d = (GridDesc<R> *)c.hostDescs;
 		long base = 0;
 		int maxSteps = 0;
 		for (int i = 0; i < n; ++i) {
@@ -394,13 +405,13 @@ static int launch_chunk(hydro_server *s, Pool &p) {
 			maxSteps = std::max(maxSteps, d[i].stepsLeft);
 			base += d[i].nItems;
 		}
-		HIPCHECK(hipMemcpyAsync(p.descs, d, descBytes, hipMemcpyHostToDevice, p.stream));
+		HIPCHECK(hipMemcpyAsync(c.descs, d, descBytes, hipMemcpyHostToDevice, p.stream));
 		const Grid &rep = s->reqs.at(active[0]).g;
 		const int o = rep.rk.order;
 		for (int j = 0; j < maxSteps; ++j) {
 			const int cur = (p.slot + j) % 3;
 			for (int st = 0; st < o; ++st)
-				if (launch_batched_stage<R>(rep, p.nvel, st, cur, (const GridDesc<R> *)p.descs, n, base, j,
+				if (launch_batched_stage<R>(rep, p.nvel, st, cur, (const GridDesc<R> *)c.descs, n, base, j,
 					p.wavesPerBlock, 1, p.stream)) return -1;
 		}
 		p.slot = (p.slot + maxSteps) % 3;
@@ -423,28 +434,28 @@ static int launch_chunk(hydro_server *s, Pool &p) {
 		r.outOff = st;
 		if (enqueue_retire(s, p, r)) return -1;
 		r.state = RETIRING;
-		p.retiring.push_back(id);
+		c.retiring.push_back(id);
 		any = true;
 	}
 	p.resident.swap(keep);
 	if (!any) return 0;
-	HIPCHECK(hipEventRecord(p.done, p.stream));
-	p.inflight = true;
-	p.started = ++s->chunks;
+	HIPCHECK(hipEventRecord(c.done, p.stream));
+	c.inflight = true;
+	c.started = ++s->chunks;
 	return 1;
 }
 
-// The chunk in flight of p has ended: the uploads' staging is released, and
+// The chunk in flight c has ended: the uploads' staging is released, and
 // finished requests are unpacked from their staging into the result and their
 // device and staging blocks released.
-static int complete_chunk(hydro_server *s, Pool &p, int *nDone) {
-	for (long long id : p.landing) {
+static int complete_chunk(hydro_server *s, Chunk &c, int *nDone) {
+	for (long long id : c.landing) {
 		Request &r = s->reqs.at(id);
 		s->pinned.release((size_t)r.upOff, r.stageBytes);
 		r.upOff = -1;
 	}
-	p.landing.clear();
-	for (long long id : p.retiring) {
+	c.landing.clear();
+	for (long long id : c.retiring) {
 		Request &r = s->reqs.at(id);
 		const char *stage = s->pinned.base + r.outOff;
 		const char *stat = stage + (size_t)r.g.Q * r.g.ps * r.g.elem;
@@ -467,8 +478,8 @@ static int complete_chunk(hydro_server *s, Pool &p, int *nDone) {
 		s->finished.push_back(id);
 		++*nDone;
 	}
-	p.retiring.clear();
-	p.inflight = false;
+	c.retiring.clear();
+	c.inflight = false;
 	return 0;
 }
 
@@ -477,26 +488,35 @@ extern "C" int hydro_server_tick(hydro_server *s, int *n_completed) {
 	int done = 0;
 	for (;;) {
 		bool moved = false;
-		for (auto &p : s->pools) {
-			if (!p.inflight) continue;
-			hipError_t e = hipEventQuery(p.done);
-			if (e == hipErrorNotReady) continue;
-			if (e != hipSuccess) return fail("chunk event: %s", hipGetErrorString(e));
-			if (complete_chunk(s, p, &done)) return -1;
-			moved = true;
-		}
-		if (admit(s, &moved)) return -1;
-		for (auto &p : s->pools) {
-			if (p.inflight || (p.joining.empty() && p.resident.empty())) continue;
-			int rc = p.cfg.precision == HYDRO_REAL_F32 ? launch_chunk<float>(s, p) : launch_chunk<double>(s, p);
-			if (rc < 0) return rc;
-			moved = moved || rc > 0;
-		}
+		for (auto &p : s->pools)
+			for (auto &c : p.chunks) {
+				if (!c.inflight) continue;
+				hipError_t e = hipEventQuery(c.done);
+				if (e == hipErrorNotReady) continue;
+				if (e != hipSuccess) return fail("chunk event: %s", hipGetErrorString(e));
+				if (complete_chunk(s, c, &done)) return -1;
+				moved = true;
+			}
+		bool admitted = false;
+		if (admit(s, &admitted)) return -1;
+		moved = moved || admitted;
+		// first one chunk for every idle pool, then, unless the next tick admits
+		// more that could join it, the one behind
+		const int deep = admitted && !s->queued.empty() ? 1 : 2;
+		for (int ahead = 0; ahead < deep; ++ahead)
+			for (auto &p : s->pools) {
+				if (p.chunks[0].inflight + p.chunks[1].inflight > ahead || (p.joining.empty() && p.resident.empty())) continue;
+				Chunk &c = p.chunks[p.chunks[0].inflight ? 1 : 0];
+				int rc = p.cfg.precision == HYDRO_REAL_F32 ? launch_chunk<float>(s, p, c) : launch_chunk<double>(s, p, c);
+				if (rc < 0) return rc;
+				moved = moved || rc > 0;
+			}
 		if (moved) break;
 		// nothing could move: wait for the chunk started first, then go again
-		Pool *first = nullptr;
+		Chunk *first = nullptr;
 		for (auto &p : s->pools)
-			if (p.inflight && (!first || p.started < first->started)) first = &p;
+			for (auto &c : p.chunks)
+				if (c.inflight && (!first || c.started < first->started)) first = &c;
 		if (!first) break;     // idle: nothing resident, nothing that fits
 		HIPCHECK(hipEventSynchronize(first->done));
 	}
@@ -539,7 +559,7 @@ extern "C" int hydro_server_info_get(hydro_server *s, hydro_server_info *info) {
 	std::memset(info, 0, sizeof *info);
 	info->queued = (int)s->queued.size();
 	for (auto &p : s->pools)
-		info->resident += (int)(p.joining.size() + p.resident.size() + p.retiring.size());
+		info->resident += (int)(p.joining.size() + p.resident.size() + p.chunks[0].retiring.size() + p.chunks[1].retiring.size());
 	info->finished = (int)s->finished.size();
 	info->pools = (int)s->pools.size();
 	info->bytes_in_use = s->arena.used;
