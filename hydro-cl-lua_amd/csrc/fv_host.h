@@ -286,31 +286,31 @@ static long grid_strips(const hydro_cfg &cfg) {
 // GLM-Maxwell FP32 512^2 14.3 (15.1), 700^2 17.4 (19.6), KH FP64 700^2 19.3 (23.5);
 // over 26 uneven shapes of all equations the rows taken were within 4 % of the
 // best of 2..16, most of them the best.
-// 3D: planes per block chunk (at most 16). Blocks are small (4 waves) and many resident
-// per CU, so the tail matters less than in 2D: keep at least 5000 blocks and,
-// among those chunk sizes, the fewest plane iterations per column (chunks that
-// divide the depth evenly, each with its 1-3 plane warm-up).
+// 3D: planes per block chunk, by the same cost over blocks of four waves; the
+// warm-up (reconstruction or jumps and one flux) and the edge pass are a plane's
+// work together. FP32 takes 2..8, FP64, with fewer blocks resident and a larger
+// state, 2..16: at 256^3 FP32 stages take 505 us at 8 planes and 515 at 16, FP64
+// 1027 and 993. us at the planes taken (against 8 at least, by an older rule):
+// 64^3 FP32 19.1 (32.7), FP64 24.8 (36.8); 128^3 FP32 76 (78); 180^3 FP64 381 (406).
 static int default_rows(const hydro_cfg &cfg) {
 	if (cfg.dim < 2) return 1;
 	const long stripsX = grid_strips(cfg), ny = cfg.size[1];
-	if (cfg.dim == 3) {
-		const int warm = cfg.plm ? 2 : (cfg.flux_limiter ? 3 : 1);
-		long W = cfg.precision == HYDRO_REAL_F32 ? Block3<float>::W : Block3<double>::W;
-		long perPlane = stripsX * ((ny + W - 1) / W);
-		long best = 8, bestCost = -1;
-		for (long r = 8; r <= EDGE_PLANES; ++r) {
-			long chunks = (cfg.size[2] + r - 1) / r;
-			if (r > 8 && perPlane * chunks < 5000) continue;
-			long cost = chunks * (r + warm);
-			if (bestCost < 0 || cost < bestCost) { best = r; bestCost = cost; }
-		}
-		return (int)best;
-	}
 	const long cus = device_cus(), occ = stage_occupancy_of(cfg, 0);
-	const bool edges = strip_edges(cfg.dim, eqn_has_source(cfg.eqn));
-	const int rMax = !edges && occ <= 2 ? 16 : 8;
 	int best = 2;
 	double bestT = -1;
+	if (cfg.dim == 3) {
+		const bool f32 = cfg.precision == HYDRO_REAL_F32;
+		const long W = f32 ? Block3<float>::W : Block3<double>::W;
+		const long perPlane = stripsX * ((ny + W - 1) / W);
+		for (int r = 2; r <= (f32 ? EDGE_PLANES / 2 : EDGE_PLANES); ++r) {
+			const long blocks = perPlane * ((cfg.size[2] + r - 1) / r);
+			const double t = march_cost((blocks + cus - 1) / cus, occ, r + 1.);
+			if (bestT < 0 || t < bestT * (1 - 1e-9)) { best = r; bestT = t; }
+		}
+		return best;
+	}
+	const bool edges = strip_edges(cfg.dim, eqn_has_source(cfg.eqn));
+	const int rMax = !edges && occ <= 2 ? 16 : 8;
 	for (int r = 2; r <= rMax; ++r) {
 		const long blocks = (stripsX * ((ny + r - 1) / r) + 3) / 4;
 		const double t = march_cost((blocks + cus - 1) / cus, occ,
