@@ -267,7 +267,7 @@ __global__ void __launch_bounds__(TOTALS_BLOCK) totals_partial_kernel(const R *U
 // as the boundary fills them: periodic/freeflow copies, mirror flips, fixed
 // values), the average and the population standard deviation over the
 // interior (the reference zeroes the ghosts for its sums and divides by the
-// interior count). Two passes (stats_kernel), FP64 compensated sums.
+// interior count). One pass (stats_kernel), FP64 compensated sums.
 // Derived Euler display variables (euler.lua:240-260) of one cell's cons
 // (rho, m, ETotal) in double: W from primFromCons (euler.cl:140-159, P by
 // calc_P, euler.cl:63-83), then the variable's formula from euler.cl:1-94.
@@ -314,15 +314,22 @@ __device__ __forceinline__ double dpp_double(double v, double none) {
 	return __builtin_bit_cast(double, q);
 }
 
-// What a pass over a field keeps: the compensated sum and the range.
+// What a field's statistics are made of: compensated sums of the values, of their
+// distances from one of them (d) and of the distances' squares (q), and the range.
 struct FieldStats {
-	KSum s;
+	KSum s, d, q;
 	double mn, mx;
 };
+__device__ __forceinline__ FieldStats stats_none() { return {{0., 0.}, {0., 0.}, {0., 0.}, INFINITY, -INFINITY}; }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ KSum ksum_step(KSum a) {
+	return ksum_merge(a, KSum{dpp_double<CTRL, ROWS>(a.s, 0.), dpp_double<CTRL, ROWS>(a.c, 0.)});
+}
 template <int CTRL, int ROWS>
 __device__ __forceinline__ void stats_step(FieldStats &a) {
-	const KSum o = {dpp_double<CTRL, ROWS>(a.s.s, 0.), dpp_double<CTRL, ROWS>(a.s.c, 0.)};
-	a.s = ksum_merge(a.s, o);
+	a.s = ksum_step<CTRL, ROWS>(a.s);
+	a.d = ksum_step<CTRL, ROWS>(a.d);
+	a.q = ksum_step<CTRL, ROWS>(a.q);
 	a.mn = fmin(a.mn, dpp_double<CTRL, ROWS>(a.mn, a.mn));
 	a.mx = fmax(a.mx, dpp_double<CTRL, ROWS>(a.mx, a.mx));
 }
@@ -341,55 +348,68 @@ __device__ __forceinline__ FieldStats stats_block(FieldStats a, FieldStats *sh) 
 	FieldStats r = sh[0];
 	for (int w = 1; w < TOTALS_BLOCK / WAVE; ++w) {
 		r.s = ksum_merge(r.s, sh[w].s);
+		r.d = ksum_merge(r.d, sh[w].d);
+		r.q = ksum_merge(r.q, sh[w].q);
 		r.mn = fmin(r.mn, sh[w].mn);
 		r.mx = fmax(r.mx, sh[w].mx);
 	}
 	return r;
 }
 
-// One of the two passes of the statistics of a field, PASS 0: range and average,
-// PASS 1: standard deviation about that average. The interior is one dense run per
+// The sum of squares about the mean from the sums about another point:
+// q - d^2 / n, in twice the precision, since it may cancel by a factor of n.
+__device__ __forceinline__ double stats_squares(const FieldStats &a, double n) {
+	const double dh = a.d.s + a.d.c, dl = (a.d.s - dh) + a.d.c;
+	const double qh = a.q.s + a.q.c, ql = (a.q.s - qh) + a.q.c;
+	const double p = dh * dh, pl = fma(dh, dh, -p) + 2. * dh * dl;
+	const double mh = p / n, ml = (fma(-mh, n, p) + pl) / n;
+	const double v = (qh - mh) + (ql - ml);
+	return v < 0. ? 0. : v;
+}
+
+// The statistics of a field in one pass: range, average, standard deviation. The
+// deviations are taken from the first interior value instead of the average, which
+// would need a pass before; their squares are summed exactly (product and its
+// rounding error). The interior is one dense run per
 // plane; ghosts can only matter to the range, and only where a face is mirrored
 // or fixed (ghosts of the others repeat interior values): those are then visited
 // on their own. The last block to finish puts the blocks' results together in
-// their order, so the result does not depend on which it is, and leaves the
-// ticket at 0; PASS 1 writes all four numbers to host memory (pinned) or out.
-// Two launches of dependent loads and reductions, bound by latency up to some
-// 10^6 cells: from call to numbers 256^2 FP64 67 -> 33, 600x400 69 -> 37, 1024^2 84 ->
-// 57 us (four launches, LDS trees of 256 and a copy back before).
-template <typename R, template <typename> class EQ, int PASS>
+// their order, so the result does not depend on which it is, leaves the
+// ticket at 0 and writes all four numbers to host memory (pinned) or out.
+// A launch of dependent loads and reductions, bound by latency up to some
+// 10^6 cells: from call to numbers 256^2 FP64 67 -> 25, 600x400 69 -> 24, 1024^2 84 -> 28 us; a
+// field of 256^3 FP32, bound by its read, 215 -> 132 (two passes, each of two launches
+// at first).
+template <typename R, template <typename> class EQ>
 __global__ void __launch_bounds__(TOTALS_BLOCK) stats_kernel(const GridDesc<R> g, int dim, int field, int ghosts,
-	double nInterior, KSum *partial, double *out, double *host, StatsPar sp)
+	double nInterior, FieldStats *partial, double *out, double *host, StatsPar sp)
 {
 	using E = EQ<R>;
 	__shared__ FieldStats sh[2][TOTALS_BLOCK / WAVE];
 	__shared__ int last;
 	const long ncell = (long)g.n[0] * g.n[1] * g.n[2];
 	const long first = (long)blockIdx.x * blockDim.x + threadIdx.x, stride = (long)gridDim.x * blockDim.x;
-	const double avg = PASS ? out[2] : 0.;
-	FieldStats a = {{0., 0.}, INFINITY, -INFINITY};
+	FieldStats a = stats_none();
 	const bool derived = E::Q == 5 && field >= HYDRO_VAR_P;
 	const R *plane = derived ? nullptr : field < E::Q ? g.U[0] + (long)field * g.ps : g.stat + (long)(field - E::Q) * g.ps;
-	for (long c = first; c < ncell; c += stride) {
-		double x;
-		if (derived) {
-			double U[5];
+	auto value = [&](long c) {
+		if (!derived) return (double)plane[c];
+		double U[5];
 #pragma unroll
-			for (int f = 0; f < 5; ++f) U[f] = (double)g.U[0][f * g.ps + c];
-			x = euler_display(sp, field, U);
-		} else {
-			x = (double)plane[c];
-		}
-		if (PASS == 0) {
-			a.mn = fmin(a.mn, x);
-			a.mx = fmax(a.mx, x);
-			a.s = ksum_add(a.s, x);
-		} else {
-			const double d = x - avg;
-			a.s = ksum_add(a.s, d * d);
-		}
+		for (int f = 0; f < 5; ++f) U[f] = (double)g.U[0][f * g.ps + c];
+		return euler_display(sp, field, U);
+	};
+	const double x0 = value(0);
+	for (long c = first; c < ncell; c += stride) {
+		const double x = value(c), d = x - x0, dd = d * d;
+		a.mn = fmin(a.mn, x);
+		a.mx = fmax(a.mx, x);
+		a.s = ksum_add(a.s, x);
+		a.d = ksum_add(a.d, d);
+		a.q = ksum_add(a.q, dd);
+		a.q.c += fma(d, d, -dd);
 	}
-	if (PASS == 0 && ghosts) {
+	if (ghosts) {
 		// ghost planes in z (whole), ghost rows in y of the others (whole), then
 		// the 2 + 2 ghosts of every interior row
 		const int gx = g.n[0] + 2 * NG, gy = dim > 1 ? g.n[1] + 2 * NG : 1;
@@ -449,35 +469,30 @@ __global__ void __launch_bounds__(TOTALS_BLOCK) stats_kernel(const GridDesc<R> g
 	}
 	a = stats_block(a, sh[0]);
 	if (threadIdx.x == 0) {
-		partial[blockIdx.x] = a.s;
-		partial[gridDim.x + blockIdx.x] = KSum{a.mn, a.mx};
+		partial[blockIdx.x] = a;
 		__threadfence();
 		last = atomicAdd(&g.dev->ticket, 1u) == gridDim.x - 1;
 	}
 	__syncthreads();
 	if (!last) return;
 	__threadfence();
-	a = FieldStats{{0., 0.}, INFINITY, -INFINITY};
+	a = stats_none();
 	for (unsigned i = threadIdx.x; i < gridDim.x; i += blockDim.x) {
-		a.s = ksum_merge(a.s, partial[i]);
-		a.mn = fmin(a.mn, partial[gridDim.x + i].s);
-		a.mx = fmax(a.mx, partial[gridDim.x + i].c);
+		const FieldStats o = partial[i];
+		a.s = ksum_merge(a.s, o.s);
+		a.d = ksum_merge(a.d, o.d);
+		a.q = ksum_merge(a.q, o.q);
+		a.mn = fmin(a.mn, o.mn);
+		a.mx = fmax(a.mx, o.mx);
 	}
 	a = stats_block(a, sh[1]);
 	if (threadIdx.x != 0) return;
 	g.dev->ticket = 0u;
-	const double sum = a.s.s + a.s.c;
-	if (PASS == 0) {
-		out[0] = a.mn;
-		out[1] = a.mx;
-		out[2] = sum / nInterior;
-	} else {
-		double *to = host ? host : out;
-		to[0] = out[0];
-		to[1] = out[1];
-		to[2] = avg;
-		to[3] = sqrt(sum / nInterior);
-	}
+	double *to = host ? host : out;
+	to[0] = a.mn;
+	to[1] = a.mx;
+	to[2] = (a.s.s + a.s.c) / nInterior;
+	to[3] = sqrt(stats_squares(a, nInterior) / nInterior);
 }
 
 } // namespace hydro

@@ -65,8 +65,8 @@ template <typename R>
 hipError_t launch_totals(const R *U, long ps, long ncell, int q, KSum *partial, int nPartial, double *out, hipStream_t s);
 
 // min, max, average, standard deviation of one field: 4 doubles to host (pinned
-// memory) where given, else to out (4 doubles on the device, used either way);
-// partial: 2 maxPartial KSums
+// memory) where given, else to out (4 doubles on the device); partial: 4
+// maxPartial KSums
 template <typename R>
 hipError_t launch_stats(int eqn, int dim, const GridDesc<R> &g, int field, KSum *partial, int maxPartial, double nInterior,
 	double *out, double *host, const double *eqnPar /* gamma, rhoMin, PMin */, hipStream_t s);
