@@ -264,11 +264,13 @@ static double march_cost(long L, long occ, double rows) {
 
 // Rows a wave marches before or beside its own: the warm-up, and in the
 // 64-column strips the edge pass, about 1.5 rows of work (.5 where four waves of
-// a block share one).
+// a block share one); the first loads of the equations with a source, of more
+// fields, are about 1.2 rows' time (GLM-Maxwell FP32 512^2: 13.6 us at 3 rows, 14.3
+// at 2).
 static double march_overhead(const hydro_cfg &cfg, bool shared) {
 	const int warm = cfg.plm ? 2 : (cfg.flux_limiter ? 3 : 1);
 	const bool edges = strip_edges(cfg.dim, eqn_has_source(cfg.eqn));
-	return warm + (!edges ? 0. : shared ? .5 : 1.5);
+	return warm + (!edges ? 1.2 : shared ? .5 : 1.5);
 }
 
 static long grid_strips(const hydro_cfg &cfg) {
