@@ -1254,13 +1254,14 @@ __device__ __forceinline__ void stage_reduce(const StageArgs<R> &a, const GridDe
 // Plain form: one grid, one wave per strip. The 2D FAST kernels of the Euler
 // equations with the Roe flux and no flux limiter take the collected Roe form
 // in their row loop (ROE_FLAGGED).
-// The FP64 form of 'plm cons' or no reconstruction without an out-of-plane
-// velocity needs about 128 registers, the most that lets a SIMD hold four
-// waves: it is held to that (the allocator takes 130 on its own, three waves).
+// The form of 'plm cons' or no reconstruction without an out-of-plane velocity is
+// held to the registers that a wave more per SIMD leaves: FP64 to 128, four waves
+// (the allocator takes 130 on its own), FP32 to 80, six (99 on its own: KH minmod
+// 4096^2 243 -> 220, 2048^2 60.7 -> 59.1, superbee 2000x1800 64.2 -> 57.5 us per stage).
 template <typename R, class E, int DIM>
 __host__ __device__ constexpr int plain_min_blocks(bool lim) {
-	return sizeof(R) == 8 && flagged_form<E, DIM>(lim) && !E::active(3) && !E::PLM_PRIM && !E::PLM_EIG && !E::PLM_CONS_FLUX
-		&& !E::PLM_ATHENA && !E::PLM_PPM && !E::PLM_EIG_PRIM && !E::PLM_EIG_PRIM_REF ? 4 : 1;
+	return flagged_form<E, DIM>(lim) && !E::active(3) && !E::PLM_PRIM && !E::PLM_EIG && !E::PLM_CONS_FLUX && !E::PLM_ATHENA
+		&& !E::PLM_PPM && !E::PLM_EIG_PRIM && !E::PLM_EIG_PRIM_REF ? (sizeof(R) == 8 ? 4 : 6) : 1;
 }
 
 template <typename R, template <typename> class EQ, int DIM, bool PLM, bool LIM, int FLIM, int SLIM>
