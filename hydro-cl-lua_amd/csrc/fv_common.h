@@ -43,13 +43,14 @@ __host__ __device__ constexpr bool tile_edges(bool source, bool lim) { return !s
 // and computes the y interfaces no row owns, so that the row waves do equal
 // work between barriers. Four waves, so that several blocks fit per CU and
 // one block's barrier waits are covered by the others' work. MIN_BLOCKS
-// bounds the registers (FP32: three blocks per CU, at most 168 VGPRs; FP64
-// takes what it needs: capped, its kernels spill).
+// bounds the registers (FP32: four blocks per CU, 128 VGPRs: the flux-limited
+// superbee and 'plm athena' kernels, at 132 on their own, 256 and 435 us against 205
+// and 359 at 200x180x160; FP64 takes what it needs: capped, its kernels spill).
 template <typename R>
 struct Block3 {
 	static constexpr int W = 3;
 	static constexpr int WAVES = W + 1;
-	static constexpr int MIN_BLOCKS = sizeof(R) == 4 ? 3 : 1;
+	static constexpr int MIN_BLOCKS = sizeof(R) == 4 ? 4 : 1;
 };
 
 // Device-resident per-solver scalars: dt minima rotate through three slots so

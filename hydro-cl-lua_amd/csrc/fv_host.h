@@ -173,6 +173,7 @@ struct Grid {
 	int dtValid;        // slot holds the min for the current state
 	int rowsPerWave;
 	int tile;           // plain 2D solver: the tile kernel in place of the marching one
+	int wholeSteps;     // plain 1D solver: a launch per step, not per stage
 	int nvel;           // Euler: velocity components that are not identically zero
 	std::vector<double> ePot;   // Euler ePot of the last upload (dynamics-neutral)
 };
@@ -281,9 +282,10 @@ static long grid_strips(const hydro_cfg &cfg) {
 // Rows per wave of the plain marching kernel: in 2D those in 2..8 of the least
 // march_cost. Short waves fill a grid that leaves SIMDs idle, long ones save
 // warm-ups, and the last round of waves should be a full one; beyond 8 nothing
-// is gained at 2048^2 and 4096^2, but a halo-strip kernel of at most 2 blocks
-// per CU takes up to 16, so that its launch can end in fewer rounds
-// (GLM-Maxwell FP64: 10 rows at 1024^2, 12 at 2048^2). us per stage at the rows
+// is gained at 2048^2 and 4096^2, but a kernel of at most 3 blocks per CU
+// takes up to 16, so that its launch can end in fewer rounds (GLM-Maxwell FP64: 10
+// rows at 1024^2, 12 at 2048^2; at 1500x1100 IEEE 'plm cons' 9 rows 93 us, 7 103,
+// HLLC 56 and 60, 'plm eig prim' 89 and 95, shallow water 10 rows 54.4, 5 57). us per stage at the rows
 // taken (against 4..8 by an older fit): shallow water 700x500 17.5 (19.3),
 // GLM-Maxwell FP32 512^2 14.3 (15.1), 700^2 17.4 (19.6), KH FP64 700^2 19.3 (23.5);
 // over 26 uneven shapes of all equations the rows taken were within 4 % of the
@@ -311,8 +313,7 @@ static int default_rows(const hydro_cfg &cfg) {
 		}
 		return best;
 	}
-	const bool edges = strip_edges(cfg.dim, eqn_has_source(cfg.eqn));
-	const int rMax = !edges && occ <= 2 ? 16 : 8;
+	const int rMax = occ <= 3 ? 16 : 8;
 	for (int r = 2; r <= rMax; ++r) {
 		const long blocks = (stripsX * ((ny + r - 1) / r) + 3) / 4;
 		const double t = march_cost((blocks + cus - 1) / cus, occ,
@@ -362,11 +363,12 @@ static long tile_blocks(const hydro_cfg &cfg) {
 // 10.6 / 10.7; at 256^2 7.8 / 10.6, 7.2 / 9.7, 7.8 / 10.7, 8.6 / 12.0, 8.1 / 9.5,
 // 7.4 / 8.8; 'plm cons' at 5.3 (512^2) 15.0 / 14.8. GLM-Maxwell FP64, twelve state
 // components in 64 bits, 8.9 / 9.9 at 1.7 (256^2), 10.8 / 10.5 at 2.5 (320^2). IEEE at
-// 14 (about 830^2): 47.1 / 50.9 at 800^2.
+// 14 (about 830^2): 47.1 / 50.9 at 800^2, but 'plm athena' 44.6 / 40.6 at 640x480.
 static bool tile_form(const hydro_cfg &cfg) {
 	if (cfg.dim != 2) return false;
 	const bool heavy = cfg.eqn == HYDRO_EQN_GLM_MAXWELL && cfg.precision == HYDRO_REAL_F64;
-	const double perCU = !cfg.fast_math ? 14. : heavy ? 2.4 : 4.5;
+	const bool cons = cfg.plm == HYDRO_PLM_NONE || cfg.plm == HYDRO_PLM_CONS;
+	const double perCU = !cfg.fast_math && cons ? 14. : heavy ? 2.4 : 4.5;
 	return (double)tile_blocks(cfg) <= perCU * (double)device_cus();
 }
 
@@ -393,6 +395,7 @@ static void grid_init(Grid &g, const hydro_cfg &cfg) {
 	g.nvel = 3;
 	g.rowsPerWave = 1;       // the caller's to set, as the form is
 	g.tile = 0;
+	g.wholeSteps = 0;
 }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
