@@ -175,6 +175,7 @@ struct Grid {
 	int tile;           // plain 2D solver: the tile kernel in place of the marching one
 	int wholeSteps;     // plain 1D solver: a launch per step, not per stage
 	int nvel;           // Euler: velocity components that are not identically zero
+	int wrote;          // the most components any launch has stored since the buffers were clear past nvel
 	std::vector<double> ePot;   // Euler ePot of the last upload (dynamics-neutral)
 };
 
@@ -393,6 +394,7 @@ static void grid_init(Grid &g, const hydro_cfg &cfg) {
 	g.slot = 0;
 	g.dtValid = 0;
 	g.nvel = 3;
+	g.wrote = 0;
 	g.rowsPerWave = 1;       // the caller's to set, as the form is
 	g.tile = 0;
 	g.wholeSteps = 0;
@@ -446,6 +448,20 @@ static void grid_bind(Grid &g, char *base) {
 	for (int i = 0; i < 3; ++i)
 		for (int j = 0; j < DT_LANES; ++j) z.dtmin[i][j] = INFINITY;
 	HIPCHECK(hipMemcpyAsync(g.dev, &z, sizeof z, hipMemcpyHostToDevice, s));
+	return 0;
+}
+
+// The stage kernels store no momentum past g.nvel, and an upload writes U[0] alone:
+// where steps end in another buffer that then becomes U[0] (forward Euler, whole 1D
+// steps), that buffer's planes past nvel still hold what a state with more
+// components left there. Clears them, once per upload that has fewer.
+[[maybe_unused]] static int clear_past_nvel(Grid &g, hipStream_t s) {
+	if (g.wrote <= g.nvel) return 0;
+	const size_t plane = (size_t)g.ps * g.elem;
+	void *other = g.ping ? g.ping : g.wholeSteps ? g.U[1] : nullptr;
+	if (other)
+		HIPCHECK(hipMemsetAsync((char *)other + (1 + g.nvel) * plane, 0, (g.wrote - g.nvel) * plane, s));
+	g.wrote = g.nvel;
 	return 0;
 }
 

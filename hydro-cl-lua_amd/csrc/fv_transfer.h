@@ -293,7 +293,8 @@ static int grid_upload(Grid &g, const void *U, size_t bytes, hipStream_t s) {
 	if (!U) return fail("NULL argument");
 	size_t need = ghosted_cells(g) * g.S * g.elem;
 	if (bytes != need) return fail("upload size %zu != %zu (numCells * numStates * sizeof(real))", bytes, need);
-	return g.elem == 8 ? grid_upload_t<double>(g, U, bytes, s) : grid_upload_t<float>(g, U, bytes, s);
+	const int rc = g.elem == 8 ? grid_upload_t<double>(g, U, bytes, s) : grid_upload_t<float>(g, U, bytes, s);
+	return rc ? rc : clear_past_nvel(g, s);
 }
 
 static int grid_download(const Grid &g, void *U, size_t bytes, hipStream_t s) {

@@ -196,6 +196,7 @@ static int solver_stage(hydro_solver *h, int s, int useSlot, double hostDt, int 
 	}
 	if (ev0) HIPCHECK(hipEventRecord(ev0, h->stream));
 	const StageKey k = stage_key(g);
+	g.wrote = std::max(g.wrote, g.nvel);
 	hipError_t e = launch_stage<R>(k, a, dim3(a.nBlocks), dim3(256), h->stream);
 	if (e != hipSuccess) return fail("stage kernel launch: %s", hipGetErrorString(e));
 	if (ev1) HIPCHECK(hipEventRecord(ev1, h->stream));
@@ -234,6 +235,7 @@ static int solver_step1d(hydro_solver *h, int steps, int useSlot, double hostDt,
 		evs->push_back(e1);
 		HIPCHECK(hipEventRecord(e0, h->stream));
 	}
+	g.wrote = std::max(g.wrote, g.nvel);
 	hipError_t e = launch_stage<R>(stage_key(g), a, dim3(a.nBlocks), dim3(WAVE * perBlock), h->stream);
 	if (e != hipSuccess) return fail("step kernel launch: %s", hipGetErrorString(e));
 	if (evs) HIPCHECK(hipEventRecord(e1, h->stream));
@@ -499,6 +501,7 @@ template <typename R>
 static int batch_stage(hydro_batch *b, int s, int cur) {
 	int nv = 0;
 	for (auto &g : b->grids) nv = std::max(nv, g.nvel);
+	for (auto &g : b->grids) g.wrote = std::max(g.wrote, nv);     // the launch stores nv of every grid
 	return launch_batched_stage<R>(b->grids[0], nv, s, cur, (const GridDesc<R> *)b->descs, (int)b->grids.size(),
 		batch_items(b), 0, b->wavesPerBlock, b->xcdRemap, b->stream);
 }
