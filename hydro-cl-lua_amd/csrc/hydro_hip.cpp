@@ -513,9 +513,10 @@ static int batch_step(hydro_batch *b, int cur) {
 	for (int s = 0; s < o; ++s)
 		if (batch_stage<R>(b, s, cur)) return -1;
 	if (o == 1) {
-		// forward Euler wrote into ping: swap every grid's buffers, which
-		// changes the descriptors of the next step
-		for (auto &g : b->grids) std::swap(g.U[0], g.ping);
+		// forward Euler wrote into ping: swap the buffers of every grid that
+		// took part, which changes the descriptors of the next step
+		for (size_t i = 0; i < b->grids.size(); ++i)
+			if (b->active[i]) std::swap(b->grids[i].U[0], b->grids[i].ping);
 		if (batch_write_descs<R>(b)) return -1;
 	}
 	return 0;

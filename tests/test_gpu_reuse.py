@@ -83,3 +83,30 @@ def test_batch_new_state_with_fewer_momenta(dim, sizes, integ):
             v.update(steps)
         for i in range(len(kws)):
             assert np.array_equal(b.download(i), fresh.download(i)), (i, steps)
+
+
+@pytest.mark.parametrize('integ', ['forward Euler', 'Runge-Kutta 2, TVD'])
+def test_batch_grid_that_sits_out(integ):
+    """an inactive grid keeps its state while the others step, and goes on from it"""
+    from hydro._cfg import make_cfg
+    from hydro.solver.batch import HipBatch
+    kws = [dict(dim=2, size=n, plm='plm cons', slope_limiter='minmod', integrator=integ, cfl=.3, boundary='freeflow',
+                precision='double', fast_math=True) for n in ((70, 33), (40, 51))]
+    cfgs = [make_cfg(**kw) for kw in kws]
+    b, alone = HipBatch(kws), HipBatch(kws[:1])
+    for i, c in enumerate(cfgs):
+        b.upload(i, _state(c, False))
+    alone.upload(0, _state(cfgs[0], False))
+    for v in (b, alone):
+        v.constrainU()
+        v.update(2)
+    for out in (1, 2, 3):
+        held = b.download(0)
+        b.setActive(0, False)
+        b.update(out)
+        assert np.array_equal(b.download(0), held), out
+        b.setActive(0, True)
+        for v in (b, alone):
+            v.update(2)
+        assert np.array_equal(b.download(0), alone.download(0)), out
+        assert b.time(0) == alone.time(0), out
