@@ -483,18 +483,29 @@ static int complete_chunk(hydro_server *s, Chunk &c, int *nDone) {
 	return 0;
 }
 
+// The chunk of p in flight that was launched first, if there is one. A pool's
+// chunks complete in this order, whatever their events say: both may end between a
+// query of the older's event and one of the younger's, and a request that the
+// older uploaded and the younger copied out may be fetched, and gone, once it is
+// finished.
+static Chunk *oldest(Pool &p) {
+	Chunk *first = nullptr;
+	for (auto &c : p.chunks)
+		if (c.inflight && (!first || c.started < first->started)) first = &c;
+	return first;
+}
+
 extern "C" int hydro_server_tick(hydro_server *s, int *n_completed) {
 	if (!s) return fail("NULL handle");
 	int done = 0;
 	for (;;) {
 		bool moved = false;
 		for (auto &p : s->pools)
-			for (auto &c : p.chunks) {
-				if (!c.inflight) continue;
-				hipError_t e = hipEventQuery(c.done);
-				if (e == hipErrorNotReady) continue;
+			while (Chunk *c = oldest(p)) {
+				hipError_t e = hipEventQuery(c->done);
+				if (e == hipErrorNotReady) break;
 				if (e != hipSuccess) return fail("chunk event: %s", hipGetErrorString(e));
-				if (complete_chunk(s, c, &done)) return -1;
+				if (complete_chunk(s, *c, &done)) return -1;
 				moved = true;
 			}
 		bool admitted = false;
@@ -506,7 +517,7 @@ extern "C" int hydro_server_tick(hydro_server *s, int *n_completed) {
 		for (int ahead = 0; ahead < deep; ++ahead)
 			for (auto &p : s->pools) {
 				if (p.chunks[0].inflight + p.chunks[1].inflight > ahead || (p.joining.empty() && p.resident.empty())) continue;
-				Chunk &c = p.chunks[p.chunks[0].inflight ? 1 : 0];
+				Chunk &c = p.chunks[p.chunks[0].inflight ? 1 : 0];      // the free one
 				int rc = p.cfg.precision == HYDRO_REAL_F32 ? launch_chunk<float>(s, p, c) : launch_chunk<double>(s, p, c);
 				if (rc < 0) return rc;
 				moved = moved || rc > 0;
@@ -515,8 +526,8 @@ extern "C" int hydro_server_tick(hydro_server *s, int *n_completed) {
 		// nothing could move: wait for the chunk started first, then go again
 		Chunk *first = nullptr;
 		for (auto &p : s->pools)
-			for (auto &c : p.chunks)
-				if (c.inflight && (!first || c.started < first->started)) first = &c;
+			if (Chunk *c = oldest(p))
+				if (!first || c->started < first->started) first = c;
 		if (!first) break;     // idle: nothing resident, nothing that fits
 		HIPCHECK(hipEventSynchronize(first->done));
 	}

@@ -358,9 +358,10 @@ int hydro_server_destroy(hydro_server *s);
  * staging than the server has. */
 int hydro_server_submit(hydro_server *s, const hydro_cfg *cfg, const void *U, size_t bytes, int nsteps,
 	long long *id);
-/* Completes the chunks that have ended (results unpacked, memory released),
- * admits, and starts the next chunk of every idle pool; it waits only when
- * none of these can happen, for the chunk started first. n_completed: requests
+/* Completes the chunks that have ended (a pool's in the order of their launch;
+ * results unpacked, memory released), admits, and starts the next chunk of every
+ * pool with fewer than two in flight; it waits only when none of these can happen,
+ * for the chunk started first. n_completed: requests
  * finished in this call. */
 int hydro_server_tick(hydro_server *s, int *n_completed);
 /* ids of finished requests whose results were not fetched yet (up to max) */

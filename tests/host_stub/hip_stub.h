@@ -1,0 +1,15 @@
+// What a CPU test puts in the place of the device (hip_stub.cpp).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <functional>
+
+#include "../../hydro-cl-lua_amd/csrc/fv_aux.h"
+#include "../../hydro-cl-lua_amd/csrc/fv_launch.h"
+
+struct StubHooks {
+	std::function<hipError_t(hipEvent_t)> query;     // hipEventQuery; unset: every event has happened
+	std::function<void(long)> give;                  // a chunk of a download is launched (its first cell)
+};
+extern StubHooks stub;
