@@ -116,7 +116,7 @@ struct GridDesc {
 // in every stored precision.
 struct EqnParD {
 	double gamma, rhoMin, PMin;   // Euler (euler.lua:192-197)
-	double eIntSafe;              // Euler: 2 PMin / (gamma - 1), the internal energy from which on P is above PMin
+	double eIntSafe;              // Euler: E - EKin from which on P is clear of PMin, 2 PMin / (gamma - 1) or more
 	double divPhi, divPsi;        // GLM-Maxwell (glm-maxwell.lua:110-111)
 	double gravity;               // shallow water (shallow-water.lua:167)
 };

@@ -61,7 +61,9 @@ static inline EqnParD eqn_par_d(const hydro_cfg &c) {
 	p.gamma = c.gamma;
 	p.rhoMin = c.rho_min;
 	p.PMin = c.P_min;
-	p.eIntSafe = 2. * c.P_min / (c.gamma - 1.);
+	// (a P above 0 is above a PMin below it; where P falls with the energy or the density
+	// may be negative, none is safe: nothing compares above a NaN)
+	p.eIntSafe = c.gamma > 1 && c.rho_min >= 0 ? std::max(0., 2. * c.P_min / (c.gamma - 1.)) : NAN;
 	p.divPhi = c.div_phi_wavespeed;
 	p.divPsi = c.div_psi_wavespeed;
 	p.gravity = c.gravity;
