@@ -22,7 +22,9 @@
 namespace hydro {
 
 // Pinned slots shared by every solver and batch of the process: at most
-// MAX_SLOTS, made as they are needed and freed with the last handle.
+// MAX_SLOTS, made as they are needed and freed with the last handle. A transfer's
+// threads keep theirs from chunk to chunk until another's wait for one (wanted), so
+// that a small transfer beside a large one waits for a chunk of it and not for all.
 class PinnedSlots {
 public:
 	static constexpr size_t SLOT = (size_t)2 << 20;
@@ -39,42 +41,60 @@ public:
 		made -= (int)idle.size();
 		idle.clear();
 	}
-	// Between 1 and `want` slots (waiting for one while all are taken); 0 if
-	// there are none and none can be made.
-	int take(int want, char **out) {
+	// A slot, in the order of the calls; nullptr if there are none and none can be
+	// made. The caller holds none itself, so that each that is taken comes back.
+	char *take() {
 		std::unique_lock<std::mutex> lock(mu);
-		for (;;) {
-			int n = 0;
-			while (n < want && !idle.empty()) {
-				out[n++] = idle.back();
-				idle.pop_back();
-			}
-			while (n < want && made < MAX_SLOTS) {
-				void *p = nullptr;
-				if (hipHostMalloc(&p, SLOT, hipHostMallocPortable) != hipSuccess || !p) {
-					(void)hipGetLastError();
-					break;
-				}
-				++made;
-				out[n++] = (char *)p;
-			}
-			if (n > 0 || made == 0) return n;
-			freed.wait(lock);
-		}
+		const long turn = last++;
+		++waiting;
+		char *p = nullptr;
+		freed.wait(lock, [&] { return turn == turns && ((p = get()) || made == 0); });
+		--waiting;
+		++turns;
+		lock.unlock();
+		freed.notify_all();
+		return p;
 	}
-	void give(char **slots, int n) {
+	// Up to `want` slots that can be had at once, if nobody waits for one.
+	int try_take(int want, char **out) {
+		std::lock_guard<std::mutex> lock(mu);
+		int n = 0;
+		while (n < want && !waiting.load() && (out[n] = get())) ++n;
+		return n;
+	}
+	bool wanted() const { return waiting.load() > 0; }
+	void give(char *const *slots, int n) {
 		{
 			std::lock_guard<std::mutex> lock(mu);
-			for (int i = 0; i < n; ++i) idle.push_back(slots[i]);
+			for (int i = 0; i < n; ++i)
+				if (slots[i]) idle.push_back(slots[i]);
 		}
 		freed.notify_all();
 	}
 
 private:
+	char *get() {
+		if (!idle.empty()) {
+			char *p = idle.back();
+			idle.pop_back();
+			return p;
+		}
+		void *p = nullptr;
+		if (made >= MAX_SLOTS) return nullptr;
+		if (hipHostMalloc(&p, SLOT, hipHostMallocPortable) != hipSuccess || !p) {
+			(void)hipGetLastError();
+			return nullptr;
+		}
+		++made;
+		return (char *)p;
+	}
+
 	std::mutex mu;
 	std::condition_variable freed;
 	std::vector<char *> idle;
 	int made = 0, handles = 0;
+	long last = 0, turns = 0;            // of take: the next to come, the one whose turn it is
+	std::atomic<int> waiting{0};
 };
 
 inline PinnedSlots &pinned_slots() {
@@ -173,14 +193,14 @@ static CellBuffer<R> cell_buffer(const Grid &g) {
 }
 
 // Moves the ghosted buffer U (host) up to or down from g's planes through the
-// slots. flags (up): what take_cells found. Returns 1 if no slot could be had
-// (nothing was moved).
+// slots, on up to 8 threads that hold up to two each. flags (up): what take_cells
+// found. Returns 1 if no slot could be had (nothing was moved).
 template <typename R, bool UP>
 static int move_cells(const Grid &g, R *U, hipStream_t s, int *flags) {
 	const size_t cellBytes = (size_t)g.S * sizeof(R);
 	const long total = (long)ghosted_cells(g);
 	const size_t bytes = (size_t)total * cellBytes;
-	constexpr size_t FLAG_BYTES = 64;
+	constexpr size_t FLAG_BYTES = 64;        // at a slot's end
 	const long maxCells = (long)((PinnedSlots::SLOT - FLAG_BYTES) / cellBytes) / CELLS_BLOCK * CELLS_BLOCK;
 	const long hw = std::max(1L, (long)std::thread::hardware_concurrency());
 	const long threads = std::max(1L, std::min({8L, hw, (long)(bytes >> 20)}));
@@ -188,17 +208,16 @@ static int move_cells(const Grid &g, R *U, hipStream_t s, int *flags) {
 	long cells = (total + 2 * threads - 1) / (2 * threads);
 	cells = std::min(maxCells, (cells + CELLS_BLOCK - 1) / CELLS_BLOCK * CELLS_BLOCK);
 	const long chunks = (total + cells - 1) / cells;
-	char *slots[PinnedSlots::MAX_SLOTS];
-	const int nSlots = pinned_slots().take((int)std::min(2 * threads, chunks), slots);
-	if (nSlots < 1) return 1;
-	const long workers = std::max(1, nSlots / 2);
+	const long workers = std::min(threads, (chunks + 1) / 2);
 	int device = 0;
 	hipError_t first = hipGetDevice(&device);
 	std::atomic<long> next{0};
-	std::atomic<int> err{(int)first};
-	int *const flagWords = (int *)(slots[0] + PinnedSlots::SLOT - FLAG_BYTES);
-	flagWords[0] = flagWords[1] = 0;
+	std::atomic<int> err{(int)first}, past{0}, outOfPlane{0};
 	const CellBuffer<R> shape = cell_buffer<R>(g);
+	// two of each thread; nullptr where there was none to be had, or it was given back
+	char *slots[PinnedSlots::MAX_SLOTS] = {};
+	static_assert(PinnedSlots::MAX_SLOTS >= 2 * 8, "of eight threads");
+	pinned_slots().try_take((int)std::min(2 * workers, chunks), slots);
 	auto work = [&](long w, bool ownThread) {
 		auto ok = [&](hipError_t e) {
 			int none = hipSuccess;
@@ -206,42 +225,66 @@ static int move_cells(const Grid &g, R *U, hipStream_t s, int *flags) {
 			return e == hipSuccess;
 		};
 		if (ownThread && !ok(hipSetDevice(device))) return;
-		const int nb = std::min(2, nSlots - (int)(2 * w));
-		hipEvent_t ev[2] = {nullptr, nullptr};
-		long at[2] = {-1, -1};      // the chunk each slot holds (down) or last sent (up)
-		for (int i = 0; i < nb; ++i)
-			if (!ok(hipEventCreateWithFlags(&ev[i], hipEventDisableTiming))) ev[i] = nullptr;
-		auto drain = [&](int i) {   // the slot's kernel has ended; down: its cells go to the caller
-			if (at[i] < 0) return;
-			if (ok(hipEventSynchronize(ev[i])) && !UP) {
-				const long c0 = at[i] * cells, n = std::min(cells, total - c0);
-				std::memcpy((char *)U + (size_t)c0 * cellBytes, slots[2 * w + i], (size_t)n * cellBytes);
+		struct Held {
+			char *&slot;
+			hipEvent_t ev;
+			long at;                // the chunk the slot holds (down) or last sent (up), -1 none
+			int *flag_words() const { return (int *)(slot + PinnedSlots::SLOT - FLAG_BYTES); }
+		} held[2] = {{slots[2 * w], nullptr, -1}, {slots[2 * w + 1], nullptr, -1}};
+		auto drain = [&](Held &h) {      // the slot's kernel has ended; down: its cells go to the caller
+			if (h.at < 0) return;
+			if (ok(hipEventSynchronize(h.ev))) {
+				if (UP) {
+					if (h.flag_words()[0]) past = 1;
+					if (h.flag_words()[1]) outOfPlane = 1;
+				} else {
+					const long c0 = h.at * cells, n = std::min(cells, total - c0);
+					std::memcpy((char *)U + (size_t)c0 * cellBytes, h.slot, (size_t)n * cellBytes);
+				}
 			}
-			at[i] = -1;
+			h.at = -1;
 		};
 		int i = 0;
-		while (err.load() == hipSuccess) {
+		while (err.load() == hipSuccess && next.load() < chunks) {
+			drain(held[i]);
+			if (held[i].slot && pinned_slots().wanted()) {
+				pinned_slots().give(&held[i].slot, 1);
+				held[i].slot = nullptr;
+			}
+			if (!held[i].slot) pinned_slots().try_take(1, &held[i].slot);
+			if (!held[i].slot && held[1 - i].slot) {
+				i = 1 - i;
+				drain(held[i]);
+			}
+			if (!held[i].slot) held[i].slot = pinned_slots().take();
+			if (!held[i].slot) break;
 			const long c = next.fetch_add(1);
 			if (c >= chunks) break;
-			drain(i);
+			Held &h = held[i];
+			if (!h.ev && !ok(hipEventCreateWithFlags(&h.ev, hipEventDisableTiming))) break;
 			CellBuffer<R> b = shape;
 			b.first = c * cells;
 			b.count = std::min(cells, total - b.first);
-			b.cells = (R *)slots[2 * w + i];
-			b.flags = flagWords;
+			b.cells = (R *)h.slot;
+			b.flags = h.flag_words();
+			b.flags[0] = b.flags[1] = 0;
 			if (UP) std::memcpy(b.cells, (const char *)U + (size_t)b.first * cellBytes, (size_t)b.count * cellBytes);
 			if (!ok(UP ? launch_take_cells<R>(b, s) : launch_give_cells<R>(b, s))) break;
-			if (!ok(hipEventRecord(ev[i], s))) {
+			if (!ok(hipEventRecord(h.ev, s))) {
 				ok(hipStreamSynchronize(s));     // the slot is still read or written
 				break;
 			}
-			at[i] = c;
-			i = i + 1 < nb ? i + 1 : 0;
+			h.at = c;
+			i = 1 - i;
 		}
-		drain(i);
-		drain(nb - 1 - i);
-		for (int k = 0; k < nb; ++k)
-			if (ev[k]) ignore(hipEventDestroy(ev[k]));
+		drain(held[i]);
+		drain(held[1 - i]);
+		for (Held &h : held)
+			if (h.ev) ignore(hipEventDestroy(h.ev));
+		if (pinned_slots().wanted()) {
+			pinned_slots().give(slots + 2 * w, 2);
+			slots[2 * w] = slots[2 * w + 1] = nullptr;
+		}
 	};
 	std::vector<std::thread> th;
 	th.reserve((size_t)workers);
@@ -254,12 +297,13 @@ static int move_cells(const Grid &g, R *U, hipStream_t s, int *flags) {
 	}
 	work(0, false);
 	for (auto &t : th) t.join();
-	if (flags) {
-		flags[0] = flagWords[0];
-		flags[1] = flagWords[1];
-	}
-	pinned_slots().give(slots, nSlots);
+	pinned_slots().give(slots, PinnedSlots::MAX_SLOTS);
 	if (err.load() != hipSuccess) return fail("transfer of the cons_t buffer: %s", hipGetErrorString((hipError_t)err.load()));
+	if (next.load() < chunks) return 1;      // nobody got a slot
+	if (flags) {
+		flags[0] = past.load();
+		flags[1] = outOfPlane.load();
+	}
 	return 0;
 }
 

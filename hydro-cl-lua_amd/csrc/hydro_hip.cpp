@@ -333,9 +333,11 @@ extern "C" int hydro_var_stats(hydro_solver *h, int field, double *out) {
 		return fail("field %d out of range 0..%d or HYDRO_VAR_*", field, g.Q + g.NSTAT - 1);
 	const double eqnPar[3] = {g.cfg.gamma, g.cfg.rho_min, g.cfg.P_min};
 	const double nInterior = (double)g.ncell;
-	char *slot = nullptr;        // the kernel writes its numbers here
-	const int have = pinned_slots().take(1, &slot);
-	double *host = have ? (double *)slot : nullptr;
+	// The kernel writes its numbers into a slot where one is free at once; where
+	// transfers hold them all, they are copied.
+	char *slot = nullptr;
+	pinned_slots().try_take(1, &slot);
+	double *const host = (double *)slot;
 	hipError_t e;
 	if (g.elem == 8) {
 		GridDesc<double> d;
@@ -349,11 +351,11 @@ extern "C" int hydro_var_stats(hydro_solver *h, int field, double *out) {
 			h->stream);
 	}
 	const hipError_t launched = e;
-	if (e == hipSuccess && !have)
+	if (e == hipSuccess && !host)
 		e = hipMemcpyAsync(out, h->totalsDev, sizeof(double) * 4, hipMemcpyDeviceToHost, h->stream);
 	const hipError_t done = hipStreamSynchronize(h->stream);
 	if (e == hipSuccess) e = done;
-	if (have) {
+	if (host) {
 		if (e == hipSuccess) std::memcpy(out, host, sizeof(double) * 4);
 		pinned_slots().give(&slot, 1);
 	}

@@ -60,7 +60,7 @@ hipError_t launch_fold_slot(DevScalars *, int, hipStream_t) { return hipSuccess;
 	template <> hipError_t launch_stats<R>(int, int, const GridDesc<R> &, int, KSum *, int, double, double *, double *, \
 		const double *, hipStream_t) { return hipSuccess; } \
 	template <> hipError_t launch_give_cells<R>(const CellBuffer<R> &b, hipStream_t) { \
-		if (stub.give) stub.give(b.first); return hipSuccess; } \
+		if (stub.give) stub.give(b.n[0]); return hipSuccess; } \
 	template <> hipError_t launch_take_cells<R>(const CellBuffer<R> &, hipStream_t) { return hipSuccess; }
 STUB_LAUNCHES(double)
 STUB_LAUNCHES(float)

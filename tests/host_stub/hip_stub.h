@@ -10,6 +10,6 @@
 
 struct StubHooks {
 	std::function<hipError_t(hipEvent_t)> query;     // hipEventQuery; unset: every event has happened
-	std::function<void(long)> give;                  // a chunk of a download is launched (its first cell)
+	std::function<void(int)> give;                   // a chunk of a download is launched (the grid's first size)
 };
 extern StubHooks stub;

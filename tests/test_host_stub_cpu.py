@@ -43,3 +43,8 @@ def _run(objects, name):
 def test_server_completes_chunks_in_launch_order(objects):
     r = _run(objects, 'server_order')
     assert r.returncode == 0 and 'in order' in r.stdout, r.stdout + r.stderr
+
+
+def test_transfers_share_the_slots(objects):
+    r = _run(objects, 'shared_slots')
+    assert r.returncode == 0 and 'shared' in r.stdout, r.stdout + r.stderr
