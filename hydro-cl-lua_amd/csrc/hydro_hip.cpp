@@ -132,8 +132,10 @@ extern "C" int hydro_set_launch(hydro_solver *h, int rows_per_wave, int xcd_rema
 	if (rows_per_wave < 0 || rows_per_wave > maxRows)
 		return fail("rows_per_wave %d out of range 0..%d", rows_per_wave, maxRows);
 	if (rows_per_wave > 0 && h->g.dim >= 2) {
+		// one row is the tile kernel where the grid is one of its, as get_launch
+		// says of it; more are the marching kernel's
 		h->g.rowsPerWave = rows_per_wave;
-		h->g.tile = 0;       // the caller's rows: the marching kernel
+		h->g.tile = rows_per_wave == 1 && tile_form(h->g.cfg);
 	}
 	if (xcd_remap > 0) h->xcdRemap = xcd_remap == 1;
 	return 0;

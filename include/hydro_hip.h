@@ -265,7 +265,8 @@ int hydro_sync(hydro_solver *h);
 
 /* Device timing of nsteps updates with HIP events on the solver stream.
  * total_ms: whole update loop; stage_ms: sum of the fused stage kernel
- * durations (events around each launch); n_stage_launches: their count. */
+ * durations (events around each launch); n_stage_launches: their count (1D grids
+ * that take a whole step per launch: of the steps). */
 typedef struct hydro_timing {
 	double total_ms;
 	double stage_ms;
@@ -277,9 +278,12 @@ int hydro_time_updates(hydro_solver *h, int nsteps, int per_kernel_events, hydro
 
 /* Launch shape of the fused stage kernel (no counterpart in the reference,
  * whose work sizes are fixed at gridsolver.lua:141-243): rows each 64-lane
- * wave marches, 1..32 (3D: planes per block, 1..16), and whether blocks are remapped so that
- * each XCD works on a contiguous band of strips. 0 keeps the current value.
- * Results do not depend on them. */
+ * wave marches, 1..32 (3D: planes per block, 1..16; 1D: ignored), and whether blocks
+ * are remapped so that each XCD works on a contiguous band of strips. 0 keeps the
+ * current value. By default the rows suit the grid's size; a 2D grid that does not
+ * fill the device has a kernel of its own with one row per wave, which reports 1 row
+ * and which 1 row selects (on larger grids 1 row is the marching kernel's). Setting
+ * what hydro_get_launch reports changes nothing. Results do not depend on them. */
 int hydro_set_launch(hydro_solver *h, int rows_per_wave, int xcd_remap);
 int hydro_get_launch(const hydro_solver *h, int *rows_per_wave, int *xcd_remap);
 

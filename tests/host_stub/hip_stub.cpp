@@ -49,8 +49,10 @@ hipError_t launch_reset_slots(DevScalars *, int, hipStream_t) { return hipSucces
 hipError_t launch_fold_slot(DevScalars *, int, hipStream_t) { return hipSuccess; }
 
 #define STUB_LAUNCHES(R) \
-	template <> hipError_t launch_stage<R>(const StageKey &, const StageArgs<R> &, dim3, dim3, hipStream_t) { \
-		stage_occupancy = 4; return hipSuccess; } \
+	template <> hipError_t launch_stage<R>(const StageKey &, const StageArgs<R> &a, dim3 grid, dim3, hipStream_t) { \
+		if (grid.x == 0) stage_occupancy = 4; \
+		else if (stub.stage) stub.stage({a.tile, a.steps, a.g.stripsX, a.g.rowsPerWave, a.g.nItems}); \
+		return hipSuccess; } \
 	template <> hipError_t launch_dt<R>(int, int, int, const GridArgs<R> &, hipStream_t) { return hipSuccess; } \
 	template <> hipError_t launch_constrain<R>(int, int, const GridArgs<R> &, hipStream_t) { return hipSuccess; } \
 	template <> hipError_t launch_nonfinite<R>(const R *, const R *, long, long, int, int, unsigned *, hipStream_t) { \

@@ -8,7 +8,14 @@
 #include "../../hydro-cl-lua_amd/csrc/fv_aux.h"
 #include "../../hydro-cl-lua_amd/csrc/fv_launch.h"
 
+// what a stage or step launch was asked for
+struct StubLaunch {
+	int tile, steps, stripsX, rows;
+	long items;
+};
+
 struct StubHooks {
+	std::function<void(const StubLaunch &)> stage;   // launch_stage
 	std::function<hipError_t(hipEvent_t)> query;     // hipEventQuery; unset: every event has happened
 	std::function<void(int)> give;                   // a chunk of a download is launched (the grid's first size)
 };

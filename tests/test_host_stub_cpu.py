@@ -48,3 +48,8 @@ def test_server_completes_chunks_in_launch_order(objects):
 def test_transfers_share_the_slots(objects):
     r = _run(objects, 'shared_slots')
     assert r.returncode == 0 and 'shared' in r.stdout, r.stdout + r.stderr
+
+
+def test_launch_shape_round_trip(objects):
+    r = _run(objects, 'launch_shape')
+    assert r.returncode == 0 and 'as reported' in r.stdout, r.stdout + r.stderr
