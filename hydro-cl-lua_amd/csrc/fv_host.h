@@ -567,9 +567,6 @@ static void stage_args(const Grid &g, int s, StageArgs<R> &a) {
 	}
 	a.storeD = needs_deriv(t, s) ? s : -1;
 	a.betaNew = t.b[s][s];
-	std::memcpy(a.rkAlpha, t.a, sizeof a.rkAlpha);
-	std::memcpy(a.rkBeta, t.b, sizeof a.rkBeta);
-	a.order = o;
 	a.steps = 0;
 	const hydro_cfg &c = g.cfg;
 	a.gamma = R(c.gamma);

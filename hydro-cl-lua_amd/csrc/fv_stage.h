@@ -967,6 +967,23 @@ __device__ __forceinline__ double general_rows(const StageArgs<R> &a, const Grid
 	return fw.dt(g.cflScale);
 }
 
+// dt of this step for grid g (solverbase.lua:3016): cfl * min, or a host value
+template <typename R>
+__device__ __forceinline__ double stage_dt(const StageArgs<R> &a, const GridDesc<R> &g) {
+	return a.dtSlot >= 0 ? g.cfl * read_dt_slot(g.dev, a.dtSlot) : a.hostDt;
+}
+
+// Per-grid bookkeeping done by the wave that owns the grid's first strip:
+// clear the next-but-one dt slot (first stage) and advance t (last stage).
+template <typename R>
+__device__ __forceinline__ void stage_first_strip(const StageArgs<R> &a, const GridDesc<R> &g, double dt, int lane) {
+	if (a.resetSlot >= 0) g.dev->dtmin[a.resetSlot][lane] = INFINITY;
+	if (a.advanceTime && lane == 0) {
+		g.dev->t = g.dev->t + dt;
+		g.dev->dt = dt;
+	}
+}
+
 // ------------------------------------------------------- one wave strip
 // Advances the strip (sx, sy) of grid g by one stage: 64 output columns (one
 // per lane; 1D: 60) by rowsPerWave (<= 32) rows. Returns the strip's dt minimum of the new
@@ -992,12 +1009,20 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 	constexpr bool EDGES = strip_edges(DIM, E::SOURCE);   // edge pass, else a halo
 	const int x = EDGES ? sx * STRIP_OUT + lane : sx * strip_out(false) - NG + lane;
 	const bool outLane = EDGES ? x < nx : lane >= NG && lane < WAVE - NG && x < nx;
+	// 1D: the dt's load goes out first, and is waited for behind the stencil's addresses
+	const double dtLane = DIM == 1 && a.dtSlot >= 0 ? g.dev->dtmin[a.dtSlot][lane] : 0.;
 	const Mapped mx = map_coord(x, nx, g.bc[0], g.bc[1], 0);
 	Mapped myIn;
 	myIn.idx = 0; myIn.mirror = 0; myIn.fixedFace = -1;
-	// taken here, and the first strip's bookkeeping left to the end: fewer values
-	// are held across the strip (KH FP64 28.3 -> 27.9 us at 1024^2, 93 -> 90 at 2048^2)
-	dt = stage_dt(a, g);
+	// taken here, and in 2D the first strip's bookkeeping left to the end: fewer values
+	// are held across the strip (KH FP64 28.3 -> 27.9 us at 1024^2, 93 -> 90 at 2048^2).
+	// A 1D launch lasts as long as one strip: there its load goes out with the others.
+	if constexpr (DIM == 1) {
+		dt = a.dtSlot >= 0 ? g.cfl * wave_min(dtLane) : a.hostDt;
+		if (sx == 0) stage_first_strip(a, g, dt, lane);
+	} else {
+		dt = stage_dt(a, g);
+	}
 	const R rdt = R(dt);
 	const R dt_dx0 = rdt / g.dx[0];
 	const R dt_dx1 = DIM >= 2 ? rdt / g.dx[1] : R(0);
@@ -1223,23 +1248,6 @@ __device__ __forceinline__ double stage_strip(const StageArgs<R> &a, const GridD
 	return a.reduceSlot >= 0 ? fw.dt(g.cflScale) : INFINITY;
 }
 
-// dt of this step for grid g (solverbase.lua:3016): cfl * min, or a host value
-template <typename R>
-__device__ __forceinline__ double stage_dt(const StageArgs<R> &a, const GridDesc<R> &g) {
-	return a.dtSlot >= 0 ? g.cfl * read_dt_slot(g.dev, a.dtSlot) : a.hostDt;
-}
-
-// Per-grid bookkeeping done by the wave that owns the grid's first strip:
-// clear the next-but-one dt slot (first stage) and advance t (last stage).
-template <typename R>
-__device__ __forceinline__ void stage_first_strip(const StageArgs<R> &a, const GridDesc<R> &g, double dt, int lane) {
-	if (a.resetSlot >= 0) g.dev->dtmin[a.resetSlot][lane] = INFINITY;
-	if (a.advanceTime && lane == 0) {
-		g.dev->t = g.dev->t + dt;
-		g.dev->dt = dt;
-	}
-}
-
 template <typename R>
 __device__ __forceinline__ void stage_reduce(const StageArgs<R> &a, const GridDesc<R> &g, double dtLocal, long item,
 	int lane)
@@ -1285,7 +1293,7 @@ __global__ void __launch_bounds__(256, (plain_min_blocks<R, EQ<R>, DIM>(LIM))) s
 	const bool share = DIM == 2 && strip_edges(DIM, EQ<R>::SOURCE) && a.shareEdges != 0 && blockDim.x == 256;
 	double dtLocal = stage_strip<R, EQ, DIM, PLM, LIM, FLIM, SLIM, false, RM>(a, g, sx, sy, dt, lane, edges, waveInBlock,
 		share);
-	if (item == 0) stage_first_strip(a, g, dt, lane);
+	if (DIM > 1 && item == 0) stage_first_strip(a, g, dt, lane);
 	stage_reduce(a, g, dtLocal, item, lane);
 }
 
@@ -1326,7 +1334,7 @@ __global__ void __launch_bounds__(256) stage_kernel_batch(const StageArgs<R> a)
 		const int sy = (int)((unsigned)local / (unsigned)g.stripsX);
 		double dtLocal = stage_strip<R, EQ, DIM, PLM, LIM, FLIM, SLIM, true, RM>(a, g, sx, sy, dt, lane, edges, waveInBlock,
 			false);
-		if (local == 0) stage_first_strip(a, g, dt, lane);
+		if (DIM > 1 && local == 0) stage_first_strip(a, g, dt, lane);
 		stage_reduce(a, g, dtLocal, local, lane);
 	}
 }

@@ -100,7 +100,7 @@ __device__ __forceinline__ void ghost_lanes(const GridDesc<R> &g, const Mapped &
 }
 
 template <typename R, template <typename> class EQ, bool PLM, bool LIM, int FLIM, int SLIM>
-__global__ void __launch_bounds__(WAVE * STEP1D_WAVES) step1d_kernel(const StageArgs<R> a)
+__global__ void __launch_bounds__(WAVE * STEP1D_WAVES) step1d_kernel(const StepArgs<R> a)
 {
 	using E = EQ<R>;
 	using C = Cell<R, E>;
@@ -130,7 +130,8 @@ __global__ void __launch_bounds__(WAVE * STEP1D_WAVES) step1d_kernel(const Stage
 	load_cell<R, E>(g, src, m, m1, U);
 	double dt = stage_dt(a, g);
 	double t = 0.;
-	if (a.advanceTime) t = g.dev->t;
+	if (oneBlock && a.advanceTime) t = g.dev->t;
+	if (!oneBlock && item == 0) stage_first_strip(a, g, dt, lane);
 	double newDt = INFINITY;           // the block's dt minimum of the last state
 
 	for (int step = 0; step < a.steps; ++step) {
@@ -203,7 +204,6 @@ __global__ void __launch_bounds__(WAVE * STEP1D_WAVES) step1d_kernel(const Stage
 				for (int j = 0; j < Q; ++j)
 					if (E::active(j)) to[j * g.ps + x] = U.v[j];
 			}
-			if (item == 0) stage_first_strip(a, g, dt, lane);
 			if (a.reduceSlot >= 0) stage_reduce(a, g, fw.dt(g.cflScale), item, lane);
 			return;
 		}

@@ -72,9 +72,11 @@ struct hydro_solver {
 // 1D grids that take several whole steps per launch, in one block
 static bool one_block(const Grid &g) { return g.n[0] <= step1d_out(g.rk.order) * STEP1D_WAVES; }
 
-// 1D grids whose steps are one launch each (fv_step1d.h). A step of one stage gains
-// nothing by it, and loses where its waves, three to a SIMD, no longer start at once
-// (flux-limited IEEE FP64, 200000 cells: 17.3 us against 14.8).
+// 1D grids whose steps are one launch each (fv_step1d.h). A step of one stage saves no
+// launch and gains a little (us per step against the stage kernel's, 'plm cons' of
+// 1000 cells FP64 5.4 / 5.6, IEEE 6.9 / 7.05, FP32 5.2 / 5.6; of 20011 5.7 / 5.8, 7.05 /
+// 7.2, 5.4 / 5.7), until its waves, three to a SIMD, no longer start at once
+// (flux-limited IEEE FP64, 200000 cells: 17.3 / 14.8).
 static bool whole_steps(const Grid &g) {
 	return g.dim == 1 && (g.rk.order > 1 || g.n[0] <= 12L * step1d_out(1) * device_cus()) &&
 		(g.cfg.boundary[0] == HYDRO_BC_PERIODIC) == (g.cfg.boundary[1] == HYDRO_BC_PERIODIC);
@@ -212,10 +214,13 @@ template <typename R>
 static int solver_step1d(hydro_solver *h, int steps, int useSlot, double hostDt, int update, std::vector<hipEvent_t> *evs) {
 	Grid &g = h->g;
 	const int cur = g.slot, fixed = g.cfg.use_fixed_dt;
-	StageArgs<R> a;
+	StepArgs<R> a;
 	stage_args<R>(g, 0, a);
 	grid_desc<R>(g, a.g);
 	a.steps = steps;
+	a.order = g.rk.order;
+	std::memcpy(a.rkAlpha, g.rk.a, sizeof a.rkAlpha);
+	std::memcpy(a.rkBeta, g.rk.b, sizeof a.rkBeta);
 	a.src = 0;
 	a.out = g.rk.order == 1 ? -1 : 1;      // the other buffer: neighbours read this one
 	if (useSlot) a.dtSlot = cur;

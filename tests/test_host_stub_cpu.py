@@ -53,3 +53,8 @@ def test_transfers_share_the_slots(objects):
 def test_launch_shape_round_trip(objects):
     r = _run(objects, 'launch_shape')
     assert r.returncode == 0 and 'as reported' in r.stdout, r.stdout + r.stderr
+
+
+def test_launches_of_1d_steps(objects):
+    r = _run(objects, 'launch_1d')
+    assert r.returncode == 0 and 'as ruled' in r.stdout, r.stdout + r.stderr
