@@ -471,15 +471,17 @@ __device__ __forceinline__ void iface_flux(const typename E::Par &p, const Iface
 // the collected form only and reports per lane whether the interface is
 // regular, so that the wave leaves its row loop at the first row with an
 // irregular interface and does the rest of its strip cell by cell, each cell's
-// four interfaces from cells of its own loading (face_difference, ROE_INLINE).
+// interfaces from cells of its own loading (general_rows, ROE_INLINE).
 // Either way each interface's form depends on its own states only, so a grid
 // advances to the same bits whatever its strips' heights and whether it runs
 // alone or batched. With both forms in the row loop the FP64 kernel needs 186
 // VGPRs (2 waves per SIMD) in place of 128 (4); after the loop, with nothing
-// of its pipeline alive, the general form fits in what the loop has. (A second
-// launch per stage used to finish such strips: 2.7 us even when there was
+// of its pipeline alive, the general form takes what the loop has, but for 3
+// registers that spill, outside the rows (FP64 at 128; FP32 at 80: none). As a function
+// out of line it took 248, with a copy of the launch's arguments in scratch. (A second
+// launch per stage used to finish such strips: 2.7 us of a stage even when there was
 // none.)
-enum { ROE_GENERAL = 0, ROE_INLINE = 1, ROE_FLAGGED = 2 };
+enum { ROE_INLINE = 1, ROE_FLAGGED = 2 };
 
 template <class E>
 __host__ __device__ constexpr bool roe_collected(bool lim) {
@@ -898,27 +900,29 @@ __device__ __forceinline__ void line_flux(const typename E::Par &par, int slim, 
 	for (int j = 0; j < E::Q; ++j) Fa[j] = fluxOn ? F[j] * aov : R(0);
 }
 
-// The difference of the fluxes on the two faces of this lane's cell (x, y)
-// along axis S, from cells loaded for this lane alone.
+// The flux, times its area factor, on the lower face along axis S of cell (x, y), from
+// cells loaded for this lane alone.
 template <typename R, class E, int S, bool PLM, int SLIM>
-__device__ __forceinline__ void face_difference(const typename E::Par &par, int slim, const GridDesc<R> &g,
-	const R *src, int x, int y, R dt_dx, R *d)
+__device__ __forceinline__ void face_flux(const typename E::Par &par, int slim, const GridDesc<R> &g, const R *src,
+	int x, int y, R dt_dx, R *Fa)
 {
-#pragma unroll 1
-	for (int side = 0; side < 2; ++side) {
-		Cell<R, E> c[4];
+	Cell<R, E> c[4];
+	Mapped mx[4], my[4];
+	bool plain = true;
 #pragma unroll
-		for (int k = 0; k < 4; ++k) {
-			const int i = side + k - 2;
-			const Mapped mx = map_coord(S == 0 ? x + i : x, g.n[0], g.bc[0], g.bc[1], 0);
-			const Mapped my = map_coord(S == 1 ? y + i : y, g.n[1], g.bc[2], g.bc[3], 2);
-			load_cell<R, E>(g, src, mx, my, c[k]);
-		}
-		R Fa[E::Q];
-		line_flux<R, E, S, PLM, SLIM>(par, slim, c, dt_dx, flux_on<E>(g, S), flux_aov<E, false>(g, S), Fa);
-#pragma unroll
-		for (int j = 0; j < E::Q; ++j) d[j] = side ? Fa[j] - d[j] : Fa[j];
+	for (int k = 0; k < 4; ++k) {
+		mx[k] = map_coord(S == 0 ? x + k - 2 : x, g.n[0], g.bc[0], g.bc[1], 0);
+		my[k] = map_coord(S == 1 ? y + k - 2 : y, g.n[1], g.bc[2], g.bc[3], 2);
+		plain = plain && mx[k].fixedFace < 0 && !mx[k].mirror && my[k].fixedFace < 0 && !my[k].mirror;
 	}
+	if (wave_all(plain)) {
+#pragma unroll
+		for (int k = 0; k < 4; ++k) load_plain<R, E>(g, src, (long)my[k].idx * g.step1 + mx[k].idx, c[k]);
+	} else {
+#pragma unroll
+		for (int k = 0; k < 4; ++k) load_cell<R, E>(g, src, mx[k], my[k], c[k]);
+	}
+	line_flux<R, E, S, PLM, SLIM>(par, slim, c, dt_dx, flux_on<E>(g, S), flux_aov<E, false>(g, S), Fa);
 }
 
 // The launch's arguments, or a grid's description, under a pointer of its own:
@@ -937,7 +941,11 @@ __device__ __forceinline__ const StageArgs<R> &kernel_args_again() {
 }
 
 // Rows y .. y1-1 of a strip's column x (this lane's) in the general form; returns
-// their dt.
+// their dt. Three interfaces a cell, the fourth kept from the row before, and cells
+// away from the faces loaded plainly: us per stage of FP64 'plm prim' with a tenth (half) of
+// the columns near vacuum, against four and mapped loads, 1024^2 93 -> 76 (114 -> 89),
+// 2048^2 287 -> 234 (302 -> 242); without a reconstruction 2048^2 163 -> 151 (178 -> 162).
+// The second launch took 77 (181), 238 (631), and 163 (514).
 template <typename R, template <typename> class EQ, int DIM, bool PLM, int SLIM>
 __device__ __forceinline__ double general_rows(const StageArgs<R> &a, const GridDesc<R> &g, int x, int y, int y1,
 	double dt)
@@ -951,14 +959,22 @@ __device__ __forceinline__ double general_rows(const StageArgs<R> &a, const Grid
 	const R dt_dx0 = R(dt) / g.dx[0], dt_dx1 = R(dt) / g.dx[1];
 	FastestOf<R, E, DIM> fw;
 	if (x < g.n[0]) {
+		R below[Q];            // the flux on the row's lower face, the one above's of the row before
+		face_flux<R, E, 1, PLM, SLIM>(par, a.limiter, g, src, x, y, dt_dx1, below);
 		for (; y < y1; ++y) {
-			R d[Q], deriv[Q];
-			face_difference<R, E, 0, PLM, SLIM>(par, a.limiter, g, src, x, y, dt_dx0, d);
+			R Fa[Q], deriv[Q];
+#pragma unroll 1
+			for (int side = 0; side < 2; ++side) {
+				face_flux<R, E, 0, PLM, SLIM>(par, a.limiter, g, src, x + side, y, dt_dx0, Fa);
 #pragma unroll
-			for (int j = 0; j < Q; ++j) deriv[j] = R(0) - d[j];
-			face_difference<R, E, 1, PLM, SLIM>(par, a.limiter, g, src, x, y, dt_dx1, d);
+				for (int j = 0; j < Q; ++j) deriv[j] = side ? R(0) - (Fa[j] - deriv[j]) : Fa[j];
+			}
+			face_flux<R, E, 1, PLM, SLIM>(par, a.limiter, g, src, x, y + 1, dt_dx1, Fa);
 #pragma unroll
-			for (int j = 0; j < Q; ++j) deriv[j] = deriv[j] - d[j];
+			for (int j = 0; j < Q; ++j) {
+				deriv[j] = deriv[j] - (Fa[j] - below[j]);
+				below[j] = Fa[j];
+			}
 			Cell<R, E> U;
 			load_plain<R, E>(g, src, (long)y * g.step1 + x, U);
 			finish_cell<R, E, DIM>(a, g, (long)y * g.step1 + x, U, deriv, dt, out, storeD, fw);
@@ -1262,14 +1278,18 @@ __device__ __forceinline__ void stage_reduce(const StageArgs<R> &a, const GridDe
 // Plain form: one grid, one wave per strip. The 2D FAST kernels of the Euler
 // equations with the Roe flux and no flux limiter take the collected Roe form
 // in their row loop (ROE_FLAGGED).
-// The form of 'plm cons' or no reconstruction without an out-of-plane velocity is
-// held to the registers that a wave more per SIMD leaves: FP64 to 128, four waves
+// Without an out-of-plane velocity, some of these are held to the registers that a
+// wave more per SIMD leaves: 'plm cons' or no reconstruction FP64 to 128, four waves
 // (the allocator takes 130 on its own), FP32 to 80, six (99 on its own: KH minmod
-// 4096^2 243 -> 220, 2048^2 60.7 -> 59.1, superbee 2000x1800 64.2 -> 57.5 us per stage).
+// 4096^2 243 -> 220, 2048^2 60.7 -> 59.1, superbee 2000x1800 64.2 -> 57.5 us per stage);
+// 'plm prim' and 'plm cons with flux' FP32 to 96, five (97 on its own with the runtime
+// limiters: 2048^2 van Leer 105.9 and 104.6 us at four).
 template <typename R, class E, int DIM>
 __host__ __device__ constexpr int plain_min_blocks(bool lim) {
-	return flagged_form<E, DIM>(lim) && !E::active(3) && !E::PLM_PRIM && !E::PLM_EIG && !E::PLM_CONS_FLUX && !E::PLM_ATHENA
-		&& !E::PLM_PPM && !E::PLM_EIG_PRIM && !E::PLM_EIG_PRIM_REF ? (sizeof(R) == 8 ? 4 : 6) : 1;
+	if (!flagged_form<E, DIM>(lim) || E::active(3)) return 1;
+	if (E::PLM_PRIM || E::PLM_CONS_FLUX) return sizeof(R) == 8 ? 1 : 5;
+	const bool cons = !E::PLM_EIG && !E::PLM_ATHENA && !E::PLM_PPM && !E::PLM_EIG_PRIM && !E::PLM_EIG_PRIM_REF;
+	return !cons ? 1 : sizeof(R) == 8 ? 4 : 6;
 }
 
 template <typename R, template <typename> class EQ, int DIM, bool PLM, bool LIM, int FLIM, int SLIM>
