@@ -260,11 +260,17 @@ static long stage_occupancy_of(const hydro_cfg &cfg, int batchWaves) {
 // waves together take 3 + k where one takes 4: a row is a chain of dependent
 // loads, square roots and divisions, and one wave alone fills a quarter of its
 // SIMD. (Measured, a row of FP32 'plm cons': 2.0, 2.65, 3.1, 3.4 us for 1..4
-// waves.)
-static double march_cost(long L, long occ, double rows) {
+// waves.) alone is that 3; 2 for the IEEE kernels of which a SIMD holds two waves at
+// most, whose division sequences fill more of it (march_alone).
+static double march_cost(long L, long occ, double rows, double alone = 3.) {
 	const long rem = L % occ;
-	return rows * ((double)(L / occ) * (3. + (double)occ) + (rem ? 3. + (double)rem : 0.));
+	return rows * ((double)(L / occ) * (alone + (double)occ) + (rem ? alone + (double)rem : 0.));
 }
+// IEEE FP64 640x480, us per stage at 3 rows (two waves a SIMD) and 5 (one): 'plm athena' 46.0
+// and 40.9, 'plm eig prim' 45.5 and 40.2, 'plm eig prim ref' 48.9 and 41.6. Over 29 such cases
+// of 420x380 .. 1500x1100 the rows taken are within 1.9 % of the best (17 % at 3), over
+// the 117 others, of more waves a SIMD, at 3 within 6.5 % (18 % at 2).
+static double march_alone(const hydro_cfg &cfg, long occ) { return !cfg.fast_math && occ <= 2 ? 2. : 3.; }
 
 // Rows a wave marches before or beside its own: the warm-up, and in the
 // 64-column strips the edge pass, about 1.5 rows of work (.5 where four waves of
@@ -320,7 +326,7 @@ static int default_rows(const hydro_cfg &cfg) {
 	for (int r = 2; r <= rMax; ++r) {
 		const long blocks = (stripsX * ((ny + r - 1) / r) + 3) / 4;
 		const double t = march_cost((blocks + cus - 1) / cus, occ,
-			r + march_overhead(cfg, stripsX % 4 == 0 && 5 * r <= WAVE));
+			r + march_overhead(cfg, stripsX % 4 == 0 && 5 * r <= WAVE), march_alone(cfg, occ));
 		if (bestT < 0 || t < bestT * (1 - 1e-9)) { best = r; bestT = t; }
 	}
 	return best;

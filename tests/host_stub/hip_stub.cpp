@@ -50,7 +50,7 @@ hipError_t launch_fold_slot(DevScalars *, int, hipStream_t) { return hipSuccess;
 
 #define STUB_LAUNCHES(R) \
 	template <> hipError_t launch_stage<R>(const StageKey &, const StageArgs<R> &a, dim3 grid, dim3, hipStream_t) { \
-		if (grid.x == 0) stage_occupancy = 4; \
+		if (grid.x == 0) stage_occupancy = stub.occupancy; \
 		else if (stub.stage) stub.stage({a.tile, a.steps, a.g.stripsX, a.g.rowsPerWave, a.g.nItems}); \
 		return hipSuccess; } \
 	template <> hipError_t launch_dt<R>(int, int, int, const GridArgs<R> &, hipStream_t) { return hipSuccess; } \

@@ -55,6 +55,23 @@ int main() {
 			REQUIRE(hydro_get_launch(h, &again, nullptr) == 0 && again == rows);
 			hydro_destroy(h);
 		}
+	// a kernel of two waves a SIMD: IEEE, whose division sequences fill more of one, takes
+	// five rows in one round where a fast one takes three in waves that run in pairs
+	stub.occupancy = 2;
+	for (int fast = 0; fast < 2; ++fast) {
+		hydro_cfg c;
+		hydro_cfg_default(&c);
+		c.dim = 2;
+		c.size[0] = 640;
+		c.size[1] = 480;
+		c.plm = HYDRO_PLM_ATHENA;
+		c.fast_math = fast;
+		hydro_solver *h = nullptr;
+		int rows = 0;
+		REQUIRE(hydro_create(&c, &h) == 0 && hydro_get_launch(h, &rows, nullptr) == 0);
+		REQUIRE(rows == (fast ? 3 : 5));
+		hydro_destroy(h);
+	}
 	std::printf("as reported\n");
 	return 0;
 }
