@@ -281,10 +281,9 @@ static int move_cells(const Grid &g, R *U, hipStream_t s, int *flags) {
 		drain(held[1 - i]);
 		for (Held &h : held)
 			if (h.ev) ignore(hipEventDestroy(h.ev));
-		if (pinned_slots().wanted()) {
-			pinned_slots().give(slots + 2 * w, 2);
-			slots[2 * w] = slots[2 * w + 1] = nullptr;
-		}
+		// now, and not when all have ended: another of these threads may wait for one
+		pinned_slots().give(slots + 2 * w, 2);
+		slots[2 * w] = slots[2 * w + 1] = nullptr;
 	};
 	std::vector<std::thread> th;
 	th.reserve((size_t)workers);
@@ -297,7 +296,7 @@ static int move_cells(const Grid &g, R *U, hipStream_t s, int *flags) {
 	}
 	work(0, false);
 	for (auto &t : th) t.join();
-	pinned_slots().give(slots, PinnedSlots::MAX_SLOTS);
+	pinned_slots().give(slots, PinnedSlots::MAX_SLOTS);      // of threads that could not be made
 	if (err.load() != hipSuccess) return fail("transfer of the cons_t buffer: %s", hipGetErrorString((hipError_t)err.load()));
 	if (next.load() < chunks) return 1;      // nobody got a slot
 	if (flags) {

@@ -19,7 +19,10 @@ const char *hipGetErrorString(hipError_t) { return "stub"; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipMalloc(void **p, size_t n) { *p = std::calloc(n, 1); return *p ? hipSuccess : hipErrorOutOfMemory; }
 hipError_t hipFree(void *p) { std::free(p); return hipSuccess; }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+	if (n >= 1 << 20 && --stub.hostBlocks < 0) return hipErrorOutOfMemory;
+	return hipMalloc(p, n);
+}
 hipError_t hipHostFree(void *p) { return hipFree(p); }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
 	std::memcpy(d, s, n);

@@ -18,6 +18,7 @@ struct StubHooks {
 	int occupancy = 4;                               // blocks of any kernel that a compute unit holds
 	std::function<void(const StubLaunch &)> stage;   // launch_stage
 	std::function<hipError_t(hipEvent_t)> query;     // hipEventQuery; unset: every event has happened
+	int hostBlocks = 1 << 30;                        // large blocks of pinned memory that can still be had
 	std::function<void(int)> give;                   // a chunk of a download is launched (the grid's first size)
 };
 extern StubHooks stub;

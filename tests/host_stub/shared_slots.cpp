@@ -51,24 +51,33 @@ int main() {
 	REQUIRE(rcA == 0);
 	REQUIRE(!statsWaited);
 	REQUIRE(!smallWaited);
-	// many at once, more threads than slots: every one ends
-	stub.give = nullptr;
-	std::vector<std::thread> th;
-	std::atomic<int> bad{0};
-	for (int k = 0; k < 24; ++k)
-		th.emplace_back([&, k] {
-			std::vector<double> U;
-			hydro_solver *h = solver(300 + k, 400, U);
-			for (int i = 0; h && i < 5; ++i)
-				if (hydro_upload_U(h, U.data(), U.size() * sizeof(double)) || hydro_download_U(h, U.data(), U.size() * sizeof(double))) ++bad;
-			if (!h) ++bad;
-			hydro_destroy(h);
-		});
-	for (auto &t : th) t.join();
-	REQUIRE(bad == 0);
+	// many at once, more threads than slots: every one ends; also with three slots in
+	// all (the others' memory cannot be had), and with none
 	hydro_destroy(a);
 	hydro_destroy(b);
 	hydro_destroy(c);
+	stub.give = nullptr;
+	for (int blocks : {1 << 30, 3, 0}) {
+		stub.hostBlocks = blocks;
+		std::vector<double> U0;
+		hydro_solver *keep = solver(16, 16, U0);     // so that the slots are freed at the end, and not between
+		std::vector<std::thread> th;
+		std::atomic<int> bad{0};
+		for (int k = 0; k < 24; ++k)
+			th.emplace_back([&, k] {
+				std::vector<double> U;
+				double four[4];
+				hydro_solver *h = solver(300 + k, 400, U);
+				for (int i = 0; h && i < 5; ++i)
+					if (hydro_upload_U(h, U.data(), U.size() * sizeof(double)) || hydro_var_stats(h, 0, four) ||
+						hydro_download_U(h, U.data(), U.size() * sizeof(double))) ++bad;
+				if (!h) ++bad;
+				hydro_destroy(h);
+			});
+		for (auto &t : th) t.join();
+		hydro_destroy(keep);
+		REQUIRE(bad == 0);
+	}
 	std::printf("shared\n");
 	return 0;
 }
