@@ -369,8 +369,8 @@ __device__ __forceinline__ double stats_squares(const FieldStats &a, double n) {
 
 // The statistics of a field in one pass: range, average, standard deviation. The
 // deviations are taken from the first interior value instead of the average, which
-// would need a pass before; their squares are summed exactly (product and its
-// rounding error). The interior is one dense run per
+// would need a pass before; their squares are summed with their rounding errors, all
+// sums compensated. The interior is one dense run per
 // plane; ghosts can only matter to the range, and only where a face is mirrored
 // or fixed (ghosts of the others repeat interior values): those are then visited
 // on their own. The last block to finish puts the blocks' results together in

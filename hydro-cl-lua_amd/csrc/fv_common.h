@@ -45,7 +45,7 @@ __host__ __device__ constexpr bool tile_edges(bool source, bool lim) { return !s
 // one block's barrier waits are covered by the others' work. MIN_BLOCKS
 // bounds the registers (FP32: four blocks per CU, 128 VGPRs: the flux-limited
 // superbee and 'plm athena' kernels, at 132 on their own, 256 and 435 us against 205
-// and 359 at 200x180x160; FP64 takes what it needs: capped, its kernels spill).
+// and 359 at 200x180x160, with 5 registers spilled, as five other FP32 kernels have; FP64 takes what it needs: capped, its kernels spill).
 template <typename R>
 struct Block3 {
 	static constexpr int W = 3;

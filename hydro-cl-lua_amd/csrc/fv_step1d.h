@@ -17,16 +17,18 @@
 // nothing leaves the CU in between.
 //
 // Per step, one launch per stage -> this: Riemann problem of 20011 cells FP32,
-// RK2-TVD 11.0 -> 6.9 us (bound by one launch and the latency of two stages); Sod on
-// 256 cells FP64 IEEE, forward Euler 6.5 -> 3.2 us in one block (the latency of one
-// stage's chain, two barriers and the dt).
+// RK2-TVD 11.0 -> 6.4 us (bound by one launch and the latency of two stages; 6.9 with
+// the first strip's bookkeeping at the end); Sod on 256 cells FP64 IEEE, forward Euler
+// 6.5 -> 3.5 us in one block (the latency of one stage's chain, two barriers and the dt).
 #pragma once
 
 #include "fv_stage.h"
 
 namespace hydro {
 
-constexpr int STEP1D_WAVES = 8;        // waves of a one-block grid at most (so that a lane has 256 registers)
+// waves of a one-block grid at most, so that a lane has 256 registers (enough but for the
+// flux-limited GLM-Maxwell FP64 forms, which spill 5 to 27)
+constexpr int STEP1D_WAVES = 8;
 
 // output cells of a wave
 __host__ __device__ constexpr int step1d_out(int order) { return WAVE - 2 * NG * order; }

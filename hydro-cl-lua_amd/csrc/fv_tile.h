@@ -178,7 +178,7 @@ __global__ void __launch_bounds__(WAVE * TILE_WAVES) stage_kernel_tile(const Sta
 
 	// ---- x on row y (lanes)
 	C Um, Up;
-	if constexpr (EDGES && (PLM || E::SOURCE)) {
+	if constexpr (EDGES && PLM) {
 		// the cells beside the strip, for lanes 0 and 63
 		C ce = c2;
 		if (lane == 0 || lane == WAVE - 1) {

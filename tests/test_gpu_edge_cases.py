@@ -3,10 +3,11 @@ expanding into vacuum (one- and two-sided vacuum Roe states, identity
 transforms below rhoMin, constrainU's density and pressure clamps), gas
 leaving a vacuum gap between two outgoing streams, and a cold gas (pressure
 below PMin, h < 1e-5 in the Roe average: Cs = 0), each in EXACT FP64, FAST
-FP64 and FP32, 1D, 2D along x and y, and 3D. The FAST Roe kernels without a
-flux limiter leave a strip, from its first row with an irregular interface
-on, to the redo kernel (fv_stage.h, ROE_FLAGGED); the other FAST kernels
-choose the Roe form per interface; so these are the cases of both paths.
+FP64 and FP32, 1D, 2D along x and y, and 3D. The 2D cases run the
+tile kernel, which chooses the Roe form per interface, as the 1D and 3D kernels do.
+The 2D marching kernels without a flux limiter do the rows of a strip from its first
+irregular interface on behind their row loop (fv_stage.h, ROE_FLAGGED,
+general_rows): the tests below that set rows per wave, and test_gpu_marching.
 
 Each case checks that the oracle's run entered the branch it is named for
 (vacuum cells, clamped densities, clamped pressures), and the HIP result
@@ -158,11 +159,11 @@ def test_edge_branches(name, init, kw, steps, branch, mode):
 
 @pytest.mark.parametrize('name,real', [('expansion-2d-x-roe', 'double'), ('streams-2d-y-roe', 'float')])
 def test_redo_same_bits_any_launch(name, real):
-    """The strips with vacuum interfaces go through the redo kernel, whose
-    rows start wherever the first irregular interface is. The Roe form is
+    """The strips with vacuum interfaces go on in the general rows, which start
+    wherever the first irregular interface is. The Roe form is
     chosen per interface and the arithmetic contracts only within a source
     expression, so the result is the same to the bit at any rows per wave and
-    in the batched kernel (with its own redo launch) as in the plain one."""
+    in the batched kernel as in the plain one."""
     from hydro.solver.batch import HipBatch
     from hydro.solver.hipfvsolver import HipFVSolver
     from hydro.init import euler as init_euler
@@ -197,7 +198,7 @@ def test_shared_edges_same_bits(real):
     of rows-per-wave interfaces fit one wave); at 13 and 16 rows, and in the
     batched kernel, each wave computes its own. The interfaces are the same
     arithmetic either way, so the results are the same to the bit, with the
-    vacuum expansion's irregular strips going through the redo kernel."""
+    vacuum expansion's irregular strips going on in the general rows."""
     from hydro.solver.batch import HipBatch
     from hydro.solver.hipfvsolver import HipFVSolver
     from hydro.init import euler as init_euler

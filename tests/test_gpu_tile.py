@@ -2,8 +2,9 @@
 default on grids that do not fill the device) and the marching kernel (rows
 per wave set) advance a grid to the same bits, whatever the scheme, type,
 boundary and size. The interfaces are the same arithmetic on the same states in
-both, so the comparison is exact. The marching kernel itself is held to the
-oracle elsewhere at these sizes."""
+both, so the comparison is exact. At these sizes it is the tile kernel that the
+other tests hold to the oracle; test_gpu_marching compares the marching kernel of
+the schemes not listed here."""
 import numpy as np
 import pytest
 
