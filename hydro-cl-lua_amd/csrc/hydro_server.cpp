@@ -483,16 +483,36 @@ static int complete_chunk(hydro_server *s, Chunk &c, int *nDone) {
 	return 0;
 }
 
-// The chunk of p in flight that was launched first, if there is one. A pool's
-// chunks complete in this order, whatever their events say: both may end between a
-// query of the older's event and one of the younger's, and a request that the
-// older uploaded and the younger copied out may be fetched, and gone, once it is
-// finished.
+// The chunk of p in flight that was launched first, if there is one.
 static Chunk *oldest(Pool &p) {
 	Chunk *first = nullptr;
 	for (auto &c : p.chunks)
 		if (c.inflight && (!first || c.started < first->started)) first = &c;
 	return first;
+}
+
+// Completes p's chunks that have ended, in the order of their launch: both may end
+// between a query of the older's event and one of the younger's, and a request that
+// the older uploaded and the younger copied out may be fetched, and gone, once it is
+// finished. They share a stream, so the younger's event tells of both, and is often
+// seen first (a burst of 14 small FP32 requests with the older's event waited for
+// 4.7 ms, 4.4 so).
+static int complete_ended(hydro_server *s, Pool &p, int *done, bool *moved) {
+	Chunk *const first = oldest(p);
+	if (!first) return 0;
+	Chunk *const second = &p.chunks[first == &p.chunks[0] ? 1 : 0];
+	Chunk *ended = nullptr;        // the last to have ended
+	for (Chunk *c : {second, first}) {
+		if (!c->inflight || ended) continue;
+		const hipError_t e = hipEventQuery(c->done);
+		if (e == hipSuccess) ended = c;
+		else if (e != hipErrorNotReady) return fail("chunk event: %s", hipGetErrorString(e));
+	}
+	if (!ended) return 0;
+	if (complete_chunk(s, *first, done)) return -1;
+	if (ended == second && complete_chunk(s, *second, done)) return -1;
+	*moved = true;
+	return 0;
 }
 
 extern "C" int hydro_server_tick(hydro_server *s, int *n_completed) {
@@ -501,13 +521,7 @@ extern "C" int hydro_server_tick(hydro_server *s, int *n_completed) {
 	for (;;) {
 		bool moved = false;
 		for (auto &p : s->pools)
-			while (Chunk *c = oldest(p)) {
-				hipError_t e = hipEventQuery(c->done);
-				if (e == hipErrorNotReady) break;
-				if (e != hipSuccess) return fail("chunk event: %s", hipGetErrorString(e));
-				if (complete_chunk(s, *c, &done)) return -1;
-				moved = true;
-			}
+			if (complete_ended(s, p, &done, &moved)) return -1;
 		bool admitted = false;
 		if (admit(s, &admitted)) return -1;
 		moved = moved || admitted;
